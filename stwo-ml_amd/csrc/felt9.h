@@ -7,8 +7,7 @@
 // accumulator with no carry handling; carries are resolved once, during the
 // reduction.  The prime has three non-zero limbs (limb 0 = 1, limb 6 =
 // 17*2^18, limb 8 = 2^19) and -p^-1 = -1 mod 2^29, so each of the nine
-// Montgomery steps is m = -t_i mod 2^29, a shift for the carry, one mad for
-// m*limb6 and one shift-add for m*limb8.
+// Montgomery digits is the negated low limb of its column and costs two mads.
 //
 // Representation rules (all values are representatives, not canonical):
 //   normalized: limbs in [0, 2^29), value below 2^261;
@@ -52,14 +51,8 @@ struct consts {
   }
 };
 
-// t (18 unnormalized 64-bit columns of a product, with 1 pre-added to columns
-// 1..9) -> t / 2^261 mod p, normalized.  Step i takes m = 2^29 - (t_i mod 2^29),
-// in [1, 2^29] and congruent to -t_i, so t_i + m = (floor(t_i / 2^29) + 1) 2^29:
-// the carry into t_(i+1) is one shift, its "+1" being the pre-added 1.  The sum
-// of the m's stays below 2^261 (1 + 2^-29), so the result is below p (1 + 2^-29)
-// + t / 2^261.
-// Hides a constant from the optimizer, so that it stays a multiplier or an
-// addend of v_mad_u64_u32 instead of being rewritten as separate shifts/adds.
+// Hides a constant from the optimizer, so that it stays a multiplier of
+// v_mad_u64_u32 instead of being rewritten as separate shifts/adds.
 template <typename T>
 GKR_HD T opaque(T v) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -67,55 +60,107 @@ GKR_HD T opaque(T v) {
 #endif
   return v;
 }
-
-GKR_HD void mont_reduce(uint64_t t[18], fe& r) {
-  const uint32_t p6 = opaque(kP6), p8 = opaque(kP8);
-#pragma unroll
-  for (int i = 0; i < 9; i++) {
-    const uint32_t m = (((uint32_t)t[i] & kMask) ^ kMask) + 1u;  // 2^29 - (t_i mod 2^29)
-    t[i + 1] += t[i] >> 29;
-    t[i + 6] += (uint64_t)m * p6;
-    t[i + 8] += (uint64_t)m * p8;
-  }
-  uint64_t c = t[9];
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    r.l[k] = (uint32_t)c & kMask;
-    c = (c >> 29) + t[10 + k];
-  }
-  r.l[8] = (uint32_t)c;
+// The same for a per-lane value: keeps sums in the written order.
+template <typename T>
+GKR_HD T in_order(T v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+v"(v));
+#endif
+  return v;
 }
 
-// Product columns start at 1 for k = 1..9 (the reduction's carry increments).
+// Products are scanned column by column (column k collects the products of
+// limbs i and k - i): one 64-bit accumulator runs through all columns, so the
+// carry from column k is the addend of column k + 1's first v_mad_u64_u32 and
+// costs no addition of its own.  Column k < 9 ends with the reduction digit
+// m_k = -(acc + e) mod 2^29, e being the 1 the digits below have carried in:
+// m_0 = 2^29 - (acc mod 2^29), and from column 1 on, where the low columns
+// always carry 1 more than acc >> 29 holds, m_k = 2^29 - 1 - (acc mod 2^29),
+// one v_bfi.  m_k enters columns k + 6 and k + 8 (limbs 6 and 8 of p; limb 0
+// cancels the column).  The carried 1 arrives in column 9, so it is added to
+// limb 0 of the result.  The sum of the m's is at most 2^261, so the result is
+// below p + t / 2^261; limb 0 is at most 2^29, the others below 2^29.
+//
+// Per product 81 (or 45 in a square) + 18 v_mad_u64_u32, 16 shifts and about 20
+// 32-bit operations.  k_merkle_level is bound by VALU issue, most of it the
+// mads.  Against unordered columns with the exact digit 2^29 - (t mod 2^29)
+// (two more operations a digit, a 64-bit addition per carry) and a partial
+// round that folded and normalized u in two passes: a partial round 333
+// instead of about 430 VALU instructions, the 275 M hashes of seven weights
+// of a Qwen2.5-14B layer 307.8 -> 243.5 ms (0.89 -> 1.13 G hashes/s).  Every
+// sum is kept in the written order (in_order): left to itself the compiler
+// adds a column's products first and the carry with a separate 64-bit
+// addition (262.8 ms).
+struct columns {
+  uint64_t acc;
+  uint32_t m[9];
+  uint32_t p6, p8;
+};
+GKR_HD void column_begin(columns& c) {
+  c.acc = 0;
+  c.p6 = opaque(kP6);
+  c.p8 = opaque(kP8);
+}
+// the reduction terms and the digit (or result limb) of column k, after its products
+template <int K>
+GKR_HD void column_end(columns& c, fe& r) {
+  if constexpr (K >= 6 && K < 15) c.acc = in_order(c.acc + (uint64_t)c.m[K - 6] * c.p6);
+  if constexpr (K >= 8) c.acc = in_order(c.acc + (uint64_t)c.m[K - 8] * c.p8);
+  if constexpr (K < 9)
+    c.m[K] = (~(uint32_t)c.acc & kMask) + (K == 0 ? 1u : 0u);
+  else
+    r.l[K - 9] = ((uint32_t)c.acc & kMask) + (K == 9 ? 1u : 0u);
+  c.acc >>= 29;
+}
+
+template <int K>
+GKR_HD void mul_columns(const fe& a, const fe& b, columns& c, fe& r) {
+  constexpr int I0 = K > 8 ? K - 8 : 0;
+  c.acc = in_order(c.acc + (uint64_t)a.l[I0] * b.l[K - I0]);  // the carry is this mad's addend
+#pragma unroll
+  for (int i = I0 + 1; i <= (K < 8 ? K : 8); i++) c.acc = in_order(c.acc + (uint64_t)a.l[i] * b.l[K - i]);
+  column_end<K>(c, r);
+  if constexpr (K < 16) mul_columns<K + 1>(a, b, c, r);
+}
+// Inputs: limbs whose pairwise products sum below 2^64 - 2^52 in every column
+// (limbs below 2^30 on both sides with top limbs below 2^29, or a normalized
+// value by limbs below 2^31).
 GKR_HD void mul(const fe& a, const fe& b, fe& r) {
-  uint64_t t[18];
-  const uint64_t one = opaque((uint64_t)1);
-#pragma unroll
-  for (int k = 0; k < 18; k++) t[k] = (k >= 1 && k <= 9) ? one : 0u;
-#pragma unroll
-  for (int i = 0; i < 9; i++)
-#pragma unroll
-    for (int j = 0; j < 9; j++) t[i + j] += (uint64_t)a.l[i] * b.l[j];
-  mont_reduce(t, r);
+  columns c;
+  fe o;
+  column_begin(c);
+  mul_columns<0>(a, b, c, o);
+  o.l[8] = (uint32_t)c.acc;
+  r = o;
 }
 
-// Off-diagonal products taken once against the doubled limbs (2 a_i < 2^31,
-// so a column stays below 4 * 2^61 + 2^60 plus the reduction terms).
+template <int K>
+GKR_HD void sqr_columns(const fe& a, const fe& d, columns& c, fe& r) {
+  constexpr int I0 = K > 8 ? K - 8 : 0;
+  c.acc = in_order(c.acc + (uint64_t)a.l[I0] * (2 * I0 < K ? d.l[K - I0] : a.l[I0]));
+#pragma unroll
+  for (int i = I0 + 1; 2 * i < K; i++) c.acc = in_order(c.acc + (uint64_t)a.l[i] * d.l[K - i]);
+  if constexpr (K % 2 == 0 && 2 * I0 < K) c.acc = in_order(c.acc + (uint64_t)a.l[K / 2] * a.l[K / 2]);
+  column_end<K>(c, r);
+  if constexpr (K < 16) sqr_columns<K + 1>(a, d, c, r);
+}
+// a^2 with d = 2a limb by limb (off-diagonal products taken once against d).
+GKR_HD void sqr2(const fe& a, const fe& d, fe& r) {
+  columns c;
+  fe o;
+  column_begin(c);
+  sqr_columns<0>(a, d, c, o);
+  o.l[8] = (uint32_t)c.acc;
+  r = o;
+}
+GKR_HD void twice(const fe& a, fe& d) {
+#pragma unroll
+  for (int i = 0; i < kLimbs; i++) d.l[i] = a.l[i] << 1;
+}
 GKR_HD void sqr(const fe& a, fe& r) {
-  uint64_t t[18];
-  const uint64_t one = opaque((uint64_t)1);
-#pragma unroll
-  for (int k = 0; k < 18; k++) t[k] = (k >= 1 && k <= 9) ? one : 0u;
-  uint32_t d[9];
-#pragma unroll
-  for (int i = 0; i < 9; i++) d[i] = a.l[i] << 1;
-#pragma unroll
-  for (int i = 0; i < 9; i++) {
-    t[2 * i] += (uint64_t)a.l[i] * a.l[i];
-#pragma unroll
-    for (int j = i + 1; j < 9; j++) t[i + j] += (uint64_t)d[i] * a.l[j];
-  }
-  mont_reduce(t, r);
+  fe d;
+  twice(a, d);
+  sqr2(a, d, r);
 }
 
 // x^3
@@ -198,8 +243,9 @@ GKR_HD void to_words(const fe& a, uint32_t w[8]) {
   }
 }
 
-// Normalized value in [0, 2^253) -> canonical residue in [0, p).
+// Value in [0, 2^253), limb 0 up to 2^29 -> canonical residue in [0, p).
 GKR_HD void canonicalize(fe& a) {
+  normalize(a);
   // subtract p up to 4 times (value < 2^253 < 5p)
 #pragma unroll
   for (int rep = 0; rep < 4; rep++) {

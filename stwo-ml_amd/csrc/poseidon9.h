@@ -11,12 +11,14 @@
 // s2): with y = x^3 and k the next partial constant,
 //   u' = 2(u + w + y),  w' = 2u,  x' = u + k - 2y,
 // which is the round s0' = 3s0 + s1 + y, s1' = s0 - s1 + y,
-// s2' = s0 + s1 + k - 2y in sum/difference coordinates.  s0 = (u + w)/2 and
-// s1 = (u - w)/2 are recovered once after the last partial round.
+// s2' = s0 + s1 + k - 2y in sum/difference coordinates.  After the first
+// partial round w = 2v with v the previous u, so a round is
+//   u' = 2(2v + u) + Y,  v' = u,  x' = u + k - Y   with Y = 2y = x^2 * 2x,
+// and s0 = u/2 + v, s1 = u/2 - v are recovered once after the last one.
 //
 // Value bounds (p ~ 2^251, R = 2^261): hash inputs below 8p; S-box inputs
 // below 9p (full) and 8p (partial) give cubes below 1.1p; u is folded below
-// 2^252 every partial round; outputs are normalized and below 5.2p.
+// 2^252 (1 + 2^-16) every partial round; outputs are normalized and below 5.2p.
 #pragma once
 #include "felt9.h"
 
@@ -61,6 +63,53 @@ GKR_HD void full_round(fe& a, fe& b, fe& c, const K& rc0, const K& rc1, const K&
   full_linear(y0, y1, y2, a, b, c);
 }
 
+// u' = 2(2v + u) + Y folded below 2^252 (1 + 2^-16) and normalized, in one
+// carry pass (u, v normalized and below 2^252 (1 + 2^-16), Y below 1.1p with
+// limb 0 up to 2^29).  The multiple of p to subtract, k = max(h - 1, 0) with
+// h = floor(u' / 2^251) up to the carries still to come, is taken from the
+// top limb before the carries; k p only touches limbs 0, 6 and 8 (k <= 15).
+// The bias 2^29 per limb, returned as 1 from the next limb, keeps every limb
+// non-negative: with it a limb is at most 8 * 2^29 - 6 and the carry into it
+// at most 7.
+GKR_HD void partial_u(const fe& u, const fe& v, const fe& Y, fe& r) {
+  uint32_t t[kLimbs];
+#pragma unroll
+  for (int k = 0; k < kLimbs; k++) t[k] = in_order((in_order((v.l[k] << 1) + u.l[k]) << 1) + Y.l[k]);  // two v_lshl_add
+  const uint32_t h = t[8] >> 19;
+  const uint32_t q = h > 0 ? h - 1 : 0;
+  t[0] -= q;
+  t[6] -= q * kP6;
+  t[8] -= q << 19;
+  uint32_t c = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const uint32_t x = t[k] + c + (k == 0 ? (1u << 29) : (1u << 29) - 1u);
+    r.l[k] = x & kMask;
+    c = x >> 29;
+  }
+  r.l[8] = t[8] + c - 1u;
+}
+// x' = u + kd - Y, normalized (kd holds 4p in limbs that dominate Y's).
+GKR_HD void partial_x(const fe& u, const fe& kd, const fe& Y, fe& x) {
+  uint32_t c = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const uint32_t t = u.l[k] + kd.l[k] + c - Y.l[k];
+    x.l[k] = t & kMask;
+    c = t >> 29;
+  }
+  x.l[8] = u.l[8] + kd.l[8] + c - Y.l[8];
+}
+// One partial round after the first: (u, v, x) -> (u', u, x'), u' in v.
+GKR_HD void partial_round(const fe& u, fe& v, fe& x, const fe& kd) {
+  fe d, x2, Y;
+  twice(x, d);
+  sqr2(x, d, x2);
+  mul(x2, d, Y);
+  partial_u(u, v, Y, v);
+  partial_x(u, kd, Y, x);
+}
+
 // out = hades([l, r, 2])[0]; l, r normalized, Montgomery, below 8p.
 GKR_HD void hash2(const fe& l, const fe& r, const hades_consts& K, fe& out) {
   fe a, b, c;
@@ -85,33 +134,33 @@ GKR_HD void hash2(const fe& l, const fe& r, const hades_consts& K, fe& out) {
   fold(u);
   normalize(w);
   add(c, K.partial0, x);
-#pragma unroll 1
-  for (int r = 0; r < 83; r++) {
+  fe v = u;
+  {
     fe y;
     cube(x, y);
-    const fe& kd = K.kd[r];
 #pragma unroll
     for (int k = 0; k < kLimbs; k++) {
       const uint32_t un = u.l[k];
       u.l[k] = 2u * (un + w.l[k] + y.l[k]);
-      w.l[k] = 2u * un;
-      x.l[k] = un + kd.l[k] - 2u * y.l[k];
+      x.l[k] = un + K.kd[0].l[k] - 2u * y.l[k];
     }
     normalize(u);
     fold(u);
     normalize(x);
   }
+#pragma unroll 1
+  for (int r = 1; r < 83; r += 2) {  // the two halves exchange the roles of u and v: no copies
+    partial_round(u, v, x, K.kd[r]);
+    partial_round(v, u, x, K.kd[r + 1]);
+  }
   c = x;
+  halve(u);
 #pragma unroll
   for (int k = 0; k < kLimbs; k++) {
-    a.l[k] = u.l[k] + w.l[k];
-    b.l[k] = u.l[k] + consts::d4(k) - w.l[k];
+    a.l[k] = u.l[k] + v.l[k];
+    b.l[k] = u.l[k] + consts::d4(k) - v.l[k];
   }
   normalize(a);
-  halve(a);
-  normalize(a);
-  normalize(b);
-  halve(b);
   normalize(b);
 #pragma unroll 1
   for (int rr = 0; rr < 3; rr++) full_round(a, b, c, K.last[rr][0], K.last[rr][1], K.last[rr][2]);
