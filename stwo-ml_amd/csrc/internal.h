@@ -33,6 +33,9 @@
 
 namespace gkr {
 struct MerkleConsts;  // merkle.h
+namespace f9 {
+struct fe;
+}
 }
 using namespace gkr;
 
@@ -240,6 +243,7 @@ struct gkr_ctx {
   std::map<uint64_t, uint32_t*> dev_tables;  // (tag << 32 | log) -> resident device copy of the table outputs
   std::map<uint64_t, felt> table_commitments;  // (tag << 32 | log) -> poseidon_hash_many([tag, log])
   MerkleConsts* merkle_consts = nullptr;  // device copy, built on first use
+  f9::fe* merkle_pairs = nullptr;         // parents of int8-range leaf pairs (merkle.h), built on first use
   bool fb_pending = false;  // f_b of the last restriction still as column-chunk partials (S_COLPART)
   uint64_t fb_rows = 0, fb_pk = 0;
   int fb_chunks = 0;
