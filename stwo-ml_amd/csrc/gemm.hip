@@ -5,14 +5,18 @@
  * C = A * B mod P for canonical M31 matrices (gemm.h).  B's digit planes (only
  * up to its highest non-zero plane) are built once per matrix and kept with
  * it; A's four planes are built per call into a context slot.  One wave per 32 x 32 tile
- * of C and K split; the splits (each at most 16384 deep, enough of them for
- * ~2048 workgroups) are added by k_gemm_reduce. */
+ * of C (int8-range operands: up to 4 x 2 tiles) and K split; the splits (each at most
+ * 16384 deep) are added by k_gemm_reduce. */
 static int digit_planes_needed(gkr_ctx* c, const uint32_t* X, uint64_t count, int* nplanes) {
   uint32_t* dmask;
   TRY(ensureT(c, S_GEMMP, 1, &dmask));
   HIP_TRY(hipMemsetAsync(dmask, 0, 4, c->stream));
-  const uint64_t blocks = std::min<uint64_t>((count + 255) / 256, 256);
-  GKR_LAUNCH(c, k_digit_mask, dim3((uint32_t)std::max<uint64_t>(blocks, 1)), dim3(256), 0, X, count, dmask);
+  const bool vec = ((uintptr_t)X & 15) == 0;
+  const dim3 grid((uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((count / (vec ? 4 : 1) + 255) / 256, 4096)));
+  if (vec)
+    GKR_LAUNCH(c, k_digit_mask<true>, grid, dim3(256), 0, X, count, dmask);
+  else
+    GKR_LAUNCH(c, k_digit_mask<false>, grid, dim3(256), 0, X, count, dmask);
   HIP_TRY(hipGetLastError());
   uint32_t mask = 0;
   HIP_TRY(hipMemcpyAsync(&mask, dmask, 4, hipMemcpyDeviceToHost, c->stream));
@@ -25,11 +29,14 @@ static int digit_planes_needed(gkr_ctx* c, const uint32_t* X, uint64_t count, in
 }
 
 static int pack_planes(gkr_ctx* c, const uint32_t* X, uint64_t outer, uint64_t K, bool kmajor, int np, int8_t* out,
-                       uint32_t* mask = nullptr) {
+                       uint32_t* mask = nullptr, uint32_t* clear = nullptr) {
   const uint64_t ntiles = (outer + kGemmTile - 1) / kGemmTile, nsteps = (K + kGemmK - 1) / kGemmK;
   const uint64_t slots = ntiles * nsteps * 64;
-  GKR_LAUNCH(c, k_digit_pack, dim3((uint32_t)((slots + 255) / 256)), dim3(256), 0, X, outer, K, kmajor, np, ntiles,
-                                                                                  nsteps, out, mask);
+  const dim3 grid((uint32_t)((slots + 255) / 256));
+  if (!kmajor && K % 4 == 0 && ((uintptr_t)X & 15) == 0)
+    GKR_LAUNCH(c, k_digit_pack<true>, grid, dim3(256), 0, X, outer, K, kmajor, np, ntiles, nsteps, out, mask, clear);
+  else
+    GKR_LAUNCH(c, k_digit_pack<false>, grid, dim3(256), 0, X, outer, K, kmajor, np, ntiles, nsteps, out, mask, clear);
   HIP_TRY(hipGetLastError());
   return GKR_OK;
 }
@@ -52,13 +59,6 @@ static int weight_planes(gkr_ctx* c, gkr_matrix* b) {
   return GKR_OK;
 }
 
-template <int PA, int PB, int U>
-static void launch_gemm(gkr_ctx* c, dim3 grid, const int8_t* ap, uint64_t apb, const uint32_t* amask,
-                        const int8_t* bp, uint64_t bpb, uint64_t m, uint64_t n, uint64_t nsteps, uint64_t rt,
-                        uint64_t ctl, uint64_t sps, uint32_t* out) {
-  GKR_LAUNCH(c, (k_gemm_m31<PA, PB, U>), grid, dim3(256), 0, ap, apb, amask, bp, bpb, m, n, nsteps, rt, ctl, sps, out);
-}
-
 static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32_t* C) {
   const uint64_t m = a->rows, k = a->cols, n = b->cols;
   TRY(weight_planes(c, b));
@@ -68,12 +68,23 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
   // A: all four planes packed (A is small) with its non-zero mask on the device;
   // B: 1 plane (int8-range weights) or 4
   const int PB = b->bnplanes == 1 ? 1 : 4;
-  void* abuf;
-  TRY(ensure(c, S_GEMMA, 256 + (size_t)4 * a_plane, &abuf));
-  uint32_t* amask = (uint32_t*)abuf;
-  int8_t* ap = (int8_t*)abuf + 256;
-  HIP_TRY(hipMemsetAsync(amask, 0, 4, c->stream));
-  TRY(pack_planes(c, a->dev, m, k, false, 4, ap, amask));
+  int8_t* ap;
+  TRY(ensureT(c, S_GEMMA, (size_t)4 * a_plane, &ap));
+  // two mask words, used in turn: the packing of one product clears the other's
+  if (!c->gemm_mask) {
+    drain(c);
+    uint32_t* w = nullptr;
+    HIP_TRY(hipMalloc(&w, 2 * sizeof(uint32_t)));
+    if (hipMemsetAsync(w, 0, 2 * sizeof(uint32_t), c->stream) != hipSuccess) {
+      (void)hipFree(w);
+      return fail(GKR_ERR_DEVICE, "clear of the digit masks failed");
+    }
+    c->gemm_mask = w;
+  }
+  uint32_t* amask = c->gemm_mask + (c->gemm_turn & 1);
+  uint32_t* next_mask = c->gemm_mask + (~c->gemm_turn & 1);
+  c->gemm_turn++;
+  TRY(pack_planes(c, a->dev, m, k, false, 4, ap, amask, next_mask));
   const int8_t* bp = b->bplanes;
   if (PB > b->bnplanes) {  // a 2- or 3-plane weight: extend with zero planes in scratch
     int8_t* ext;
@@ -83,22 +94,53 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
     bp = ext;
   }
   const uint64_t waves = rtiles * ctiles, blocks_x = (waves + 3) / 4;
-  uint64_t splits = (2048 + blocks_x - 1) / blocks_x;
+  // Int8-range operands: the wave's tiles by the rows there are (times of one
+  // product with 5120 x 13824 int8 weights, one tile per wave and 2048
+  // workgroups by K splits before -> now): 4 x 2 from 8 row tiles (m = 512:
+  // 218.5 -> 58.2 us, 1024: 397 -> 104), 2 x 2 from 4 (128 x 5120 x 5120: 42.9
+  // -> 25.0), 2 x 1 from 2 (m = 64: 48.6 -> 32.2), 1 x 1 for one (m = 1: 26.3
+  // -> 19.0).  K is split only where the tiles alone give under 576 waves, and
+  // then into about 768 waves (512 and 1024 up to 1.3 times slower for one
+  // shape or another): a split writes and reads its partial sums.
+  const int RT = rtiles >= 8 ? 4 : rtiles >= 2 ? 2 : 1, CT = rtiles >= 4 ? 2 : 1, WR = rtiles >= 4 ? 2 : 1;
+  const uint64_t rgroups = (rtiles + RT * WR - 1) / (RT * WR), cgroups = (ctiles + CT * (4 / WR) - 1) / (CT * (4 / WR));
+  const uint64_t tile_waves = (rtiles + RT - 1) / RT * ((ctiles + CT - 1) / CT);
+  uint64_t splits = PB == 1 ? (tile_waves >= 576 ? 1 : (768 + tile_waves - 1) / tile_waves)
+                            : (2048 + blocks_x - 1) / blocks_x;
   splits = std::min<uint64_t>(splits, std::max<uint64_t>(1, nsteps / 16));
   splits = std::max<uint64_t>(splits, (nsteps * kGemmK + kGemmMaxKPass - 1) / kGemmMaxKPass);
   const uint64_t sps = (nsteps + splits - 1) / splits;
   splits = (nsteps + sps - 1) / sps;
-  if (blocks_x > 0x7fffffffull || splits > 65535) return fail(GKR_ERR_INVALID, "forward GEMM: grid too large");
+  if (blocks_x > 0x7fffffffull || (cgroups + 7) / 8 * 8 * rgroups > 0x7fffffffull || nsteps > 0xffffffffull || splits > 65535)
+    return fail(GKR_ERR_INVALID, "forward GEMM: grid too large");
   uint32_t* part = C;
   if (splits > 1) TRY(ensureT(c, S_GEMMP, splits * m * n, &part));
-  const dim3 grid((uint32_t)blocks_x, (uint32_t)splits);
-  // exactly one of each pair works (the other reads the mask and returns)
   if (PB == 1) {
-    launch_gemm<1, 1, 16>(c, grid, ap, a_plane, amask, bp, b_plane, m, n, nsteps, rtiles, ctiles, sps, part);
-    launch_gemm<4, 1, 4>(c, grid, ap, a_plane, amask, bp, b_plane, m, n, nsteps, rtiles, ctiles, sps, part);
+    const dim3 g8((uint32_t)((cgroups + 7) / 8 * 8 * rgroups), (uint32_t)splits);
+    auto int8_launch = [&](auto kernel) {
+      GKR_LAUNCH(c, kernel, g8, dim3(256), 0, ap, a_plane, amask, bp, m, n, (uint32_t)nsteps, (uint32_t)rtiles,
+                 (uint32_t)ctiles, (uint32_t)rgroups, (uint32_t)cgroups, (uint32_t)sps, part);
+    };
+    if (RT == 4)
+      int8_launch(k_gemm_int8<4, 2, 2>);
+    else if (CT == 2)
+      int8_launch(k_gemm_int8<2, 2, 2>);
+    else if (RT == 2)
+      int8_launch(k_gemm_int8<2, 1, 1>);
+    else
+      int8_launch(k_gemm_int8<1, 1, 1>);
+    auto a4_launch = [&](auto kernel, uint64_t ct) {
+      GKR_LAUNCH(c, kernel, dim3((uint32_t)((rtiles * ((ctiles + ct - 1) / ct) + 3) / 4), (uint32_t)splits), dim3(256), 0,
+                 ap, a_plane, amask, bp, m, n, nsteps, rtiles, ctiles, sps, part);
+    };
+    // two column tiles per wave from 4096 tiles (128 x 1024 x 1024, 128 tiles: 17.9 us with one, 22.2 with two)
+    if (RT * CT > 1 && waves * splits >= 4096)
+      a4_launch(k_gemm_a4<2>, 2);
+    else if (RT * CT > 1)
+      a4_launch(k_gemm_a4<1>, 1);
   } else {
-    launch_gemm<1, 4, 4>(c, grid, ap, a_plane, amask, bp, b_plane, m, n, nsteps, rtiles, ctiles, sps, part);
-    launch_gemm<4, 4, 2>(c, grid, ap, a_plane, amask, bp, b_plane, m, n, nsteps, rtiles, ctiles, sps, part);
+    GKR_LAUNCH(c, k_gemm_m31, dim3((uint32_t)blocks_x, (uint32_t)splits), dim3(256), 0, ap, a_plane, amask, bp, b_plane,
+               m, n, nsteps, rtiles, ctiles, sps, part);
   }
   HIP_TRY(hipGetLastError());
   if (splits > 1) {

@@ -243,6 +243,8 @@ struct gkr_ctx {
   std::map<uint64_t, uint32_t*> dev_tables;  // (tag << 32 | log) -> resident device copy of the table outputs
   std::map<uint64_t, felt> table_commitments;  // (tag << 32 | log) -> poseidon_hash_many([tag, log])
   MerkleConsts* merkle_consts = nullptr;  // device copy, built on first use
+  uint32_t* gemm_mask = nullptr;          // forward product: A's non-zero planes, two words in turn
+  uint32_t gemm_turn = 0;
   f9::fe* merkle_pairs = nullptr;         // parents of int8-range leaf pairs (merkle.h), built on first use
   bool fb_pending = false;  // f_b of the last restriction still as column-chunk partials (S_COLPART)
   uint64_t fb_rows = 0, fb_pk = 0;

@@ -415,6 +415,7 @@ extern "C" void gkr_ctx_destroy(gkr_ctx* c) {
   for (auto& t : c->dev_tables) (void)hipFree(t.second);
   if (c->merkle_consts) (void)hipFree(c->merkle_consts);
   if (c->merkle_pairs) (void)hipFree(c->merkle_pairs);
+  if (c->gemm_mask) (void)hipFree(c->gemm_mask);
   if (c->h_res) (void)hipHostFree(c->h_res);
   c->mring.reset();  // freed with the last proof record still holding a slot
   for (int s = 0; s < H_NSLOTS; s++)

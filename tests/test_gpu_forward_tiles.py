@@ -1,0 +1,46 @@
+"""The forward product over int8-range weights around its tile shapes (csrc/gemm.h): row counts on both
+sides of each rule (1, 2, 4 and 8 row tiles of 32), ragged columns and inner sizes with and without K
+splits, and activations of one digit plane and of four.  Against exact integers."""
+import numpy as np
+import pytest
+
+import gkr_mi355x as G
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+P = G.P
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = G.Context(0)
+    yield c
+    c.close()
+
+
+def exact(a, b):
+    """A * B mod P over 16-bit halves of A, centered int8 B: every partial sum below 2^53."""
+    bc = np.where(b > P // 2, b.astype(np.int64) - P, b.astype(np.int64)).astype(np.float64)
+    lo = ((a & 0xFFFF).astype(np.float64) @ bc).astype(np.int64)
+    hi = ((a >> 16).astype(np.float64) @ bc).astype(np.int64)
+    return ((lo + (hi % P) * 65536) % P).astype(np.uint32)
+
+
+@pytest.mark.parametrize("m", [1, 32, 33, 64, 97, 128, 224, 225, 300, 513])
+@pytest.mark.parametrize("k,n", [(40, 70), (1100, 257), (3000, 31), (96, 4099)])
+def test_tile_rules(ctx, m, k, n):
+    b = O.synthetic(k, n, 1, 7)
+    b[0, 0], b[-1, -1] = 127, P - 127
+    dev = ctx.upload(b)
+    for kind in (1, 0):  # one digit plane, then four, then one again (the mask words take turns)
+        a = O.synthetic(m, k, kind, 11 + m)
+        assert np.array_equal(ctx.matmul_forward(ctx.upload(a), dev).download(), exact(a, b))
+    a = O.synthetic(m, k, 1, 12 + m)
+    assert np.array_equal(ctx.matmul_forward(ctx.upload(a), dev).download(), exact(a, b))
+
+
+def test_one_high_value_takes_the_general_path(ctx):
+    """A single entry of A outside the int8 range, in the last row."""
+    a, b = O.synthetic(300, 200, 1, 5), O.synthetic(200, 300, 1, 6)
+    a[-1, -1] = 1 << 20
+    assert np.array_equal(ctx.matmul_forward(ctx.upload(a), ctx.upload(b)).download(), exact(a, b))
