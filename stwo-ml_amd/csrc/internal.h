@@ -677,6 +677,19 @@ constexpr uint64_t kTripBig = GKR_TRIP_BIG;
 constexpr uint64_t kTripHuge = GKR_TRIP_HUGE;
 // Rounds per trip over a vector of n entries: 3 up to kTripBig, 2 up to kTripHuge, then 1.
 static inline int trip_k(uint64_t n) { return n > kTripHuge ? 1 : n > kTripBig ? 2 : 3; }
+// Trips of three rounds over kMfmaTripMin to kMfmaTripMaxN entries run on the
+// matrix cores (trip_mfma.h), whatever their length: product sumchecks plan
+// their trips with product_trip_k.  At 2^16 entries and below k_trip<0, 3> is
+// as fast (a 2^16 sumcheck 181 us with either).
+#ifndef GKR_MFMA_TRIP_MIN
+#define GKR_MFMA_TRIP_MIN (1ull << 17)
+#endif
+constexpr uint64_t kMfmaTripMin = GKR_MFMA_TRIP_MIN;
+constexpr uint64_t kMfmaTripMaxN = 1ull << 29;  // int32 sums: 2^16 x per workgroup on 1024 workgroups
+static_assert(kMfmaTripMin >= 512 && kMfmaTripMin <= 2 * kTripBig, "no trip kernel for three rounds between");
+static inline int product_trip_k(uint64_t n) {
+  return n >= kMfmaTripMin && n <= kMfmaTripMaxN ? 3 : trip_k(n);
+}
 #ifndef GKR_TRIP_MAX_BLOCKS
 #define GKR_TRIP_MAX_BLOCKS 512
 #endif
@@ -704,7 +717,7 @@ static_assert(GKR_TRIP_MAX_BLOCKS_SHORT <= kMaxPartialBlocks && GKR_TRIP_MAX_BLO
 #endif
 constexpr unsigned kTripFusedGrid = GKR_TRIP_FUSED_GRID;
 constexpr uint64_t kTripSplitLanes = 256ull * kBlock;
-std::vector<Trip> plan_trips(int T, uint64_t host_len, int k0);
+std::vector<Trip> plan_trips(int T, uint64_t host_len, int k0, int (*trip_rounds)(uint64_t) = trip_k);
 static inline int trip_nq(int kind, int K) { return kind == 2 ? (1 << K) : (1 << (2 * K)); }
 // eqlin(z, X) = (1 - z)(1 - X) + z X, the multilinear eq factor of one coordinate.
 static inline qm31 eqlin(const qm31& z, const qm31& x) {

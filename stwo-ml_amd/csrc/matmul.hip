@@ -362,7 +362,8 @@ int product_sumcheck(gkr_ctx* c, PoseidonChannel& ch, int T, const qm31* in_a, c
                             const qm31* scale3, const FirstTrip* ft) {
   const qm31 inv2 = qm31_from_m31(1u << 30);  // 2^-1 mod P
   const uint64_t pk = 1ull << T;
-  const std::vector<Trip> trips = plan_trips(T, kHostTailMM, g0 ? k0 : trip_k(1ull << T));
+  const std::vector<Trip> trips = plan_trips(T, kHostTailMM, g0 ? k0 : ft && ft->b_chunks ? trip_k(1ull << T) : product_trip_k(1ull << T),
+                                             product_trip_k);
   std::vector<qm31> chal(T);
   auto absorb = [&](int t, const qm31* sums) {
     const qm31 c0 = sums[0];

@@ -2,6 +2,7 @@
 // multi-round trip launcher shared by the layer reducers; the bandwidth
 // reference kernels.
 #include "internal.h"
+#include "trip_mfma.h"
 
 // ------------------------------------------------------------------ errors, version
 thread_local std::string g_err = "";
@@ -201,14 +202,14 @@ int make_sink(gkr_ctx* c, RoundSink* sk, int slot) {
   sk->seq = alloc_seq(&c->seq, 1);
   return GKR_OK;
 }
-std::vector<Trip> plan_trips(int T, uint64_t host_len, int k0) {
+std::vector<Trip> plan_trips(int T, uint64_t host_len, int k0, int (*trip_rounds)(uint64_t)) {
   std::vector<Trip> v;
   if (T <= 0) return v;
   int t = k0 < T ? k0 : T;
   v.push_back({0, t, 1ull << T});
   while (t < T && (1ull << (T - t)) > host_len) {
     const uint64_t n = 1ull << (T - t);
-    int k = trip_k(n);
+    int k = trip_rounds(n);
     if (k > T - t) k = T - t;
     v.push_back({t, k, n});
     t += k;
@@ -235,29 +236,21 @@ void trip_round_sum(const qm31* S, int K, int j, const qm31* r, qm31* out) {
     out[b] = qm31_add(out[b], qm31_mul(E[u], S[c]));
   }
 }
-// Launch k_trip<KIND, K> over sources sa (, sb) of length n << np with the
-// np pending challenges `pend`; folded vectors to da (, db) when given; eq
-// weights (KIND 1) from hi/lo; then the finisher into sink slot `slot`.
-template <int KIND, int K, bool SPLIT>
-static int launch_trip_k(gkr_ctx* c, const qm31* sa, const qm31* sb, uint64_t n, int np, const TripChal& al,
-                         qm31* da, qm31* db, const qm31* hi, const qm31* lo, int h, const RoundSink& sk,
-                         unsigned grid, uint64_t b_rows, int b_chunks, const TripWait& tw, CarriedFinish* carry_out,
-                         const CarriedFinish* carry_in) {
-  constexpr int NQ = TripShape<KIND, K, SPLIT>::NQ;
-  uint32_t* counter = nullptr;
-  uint32_t base = 0;
-  if (!carry_out && GKR_TRIP_FUSED && grid <= kTripFusedMax)  // one launch: the last workgroup finishes
-    TRY(arrival_counter(c, grid, &counter, &base));
+// The launches of one trip around its kernel (`kernel` queues it): the wait
+// for its challenges when launched ahead, then the finisher into its sink, or
+// its rows handed to the next kernel of the chain.
+template <int NQ, typename F>
+static int launch_trip_chain(gkr_ctx* c, const RoundSink& sk, unsigned grid, bool in_kernel_finish, const TripWait& tw,
+                             CarriedFinish* carry_out, const CarriedFinish* carry_in, F kernel) {
   if (tw.chal) {  // launched ahead: the challenges arrive through the mailbox
     CarriedFinish none;
     memset(&none, 0, sizeof none);
     GKR_LAUNCH(c, k_mailbox_wait, dim3(1), dim3(kWaitBlock), 0, tw, carry_in ? *carry_in : none);
     TRY(check_launch(c));
   }
-  GKR_LAUNCH(c, (k_trip<KIND, K, SPLIT>), dim3(grid), dim3(kBlock), 0, sa, sb, n, np, al, da, db, hi, lo, h,
-                     sk, counter, base, b_rows, b_chunks, tw);
+  kernel();
   TRY(check_launch(c));
-  if (counter) return GKR_OK;
+  if (in_kernel_finish) return GKR_OK;
   if (carry_out) {  // the next kernel of the chain adds the rows
     carry_out->sk = sk;
     carry_out->nblocks = grid;
@@ -268,6 +261,48 @@ static int launch_trip_k(gkr_ctx* c, const qm31* sa, const qm31* sb, uint64_t n,
   }
   GKR_LAUNCH(c, k_finish_wide<NQ>, dim3(1), dim3(kFinishBlock), 0, sk, grid);
   return check_launch(c);
+}
+// Launch k_trip<KIND, K> over sources sa (, sb) of length n << np with the
+// np pending challenges `pend`; folded vectors to da (, db) when given; eq
+// weights (KIND 1) from hi/lo; then the finisher into sink slot `slot`.
+template <int KIND, int K, bool SPLIT>
+static int launch_trip_k(gkr_ctx* c, const qm31* sa, const qm31* sb, uint64_t n, int np, const TripChal& al,
+                         qm31* da, qm31* db, const qm31* hi, const qm31* lo, int h, const RoundSink& sk,
+                         unsigned grid, uint64_t b_rows, int b_chunks, const TripWait& tw, CarriedFinish* carry_out,
+                         const CarriedFinish* carry_in) {
+  uint32_t* counter = nullptr;
+  uint32_t base = 0;
+  if (!carry_out && GKR_TRIP_FUSED && grid <= kTripFusedMax)  // one launch: the last workgroup finishes
+    TRY(arrival_counter(c, grid, &counter, &base));
+  return launch_trip_chain<TripShape<KIND, K, SPLIT>::NQ>(c, sk, grid, counter != nullptr, tw, carry_out, carry_in, [&] {
+    GKR_LAUNCH(c, (k_trip<KIND, K, SPLIT>), dim3(grid), dim3(kBlock), 0, sa, sb, n, np, al, da, db, hi, lo, h,
+                       sk, counter, base, b_rows, b_chunks, tw);
+  });
+}
+#ifndef GKR_MFMA_TRIP_BLOCKS
+#define GKR_MFMA_TRIP_BLOCKS 512
+#endif
+// two workgroups per CU (its registers allow no more); a large grid only where a
+// workgroup would exceed kMfmaTripMaxX
+constexpr uint64_t kMfmaTripBlocks = GKR_MFMA_TRIP_BLOCKS;
+// The same for k_trip_mfma<KIND, NP> (three rounds).
+template <int KIND>
+static int launch_trip_mfma(gkr_ctx* c, const qm31* sa, const qm31* sb, uint64_t n, int np, const TripChal& al,
+                            qm31* da, qm31* db, const qm31* hi, const qm31* lo, int h, const RoundSink& sk,
+                            unsigned grid, const TripWait& tw, CarriedFinish* carry_out, const CarriedFinish* carry_in) {
+  return launch_trip_chain<64>(c, sk, grid, false, tw, carry_out, carry_in, [&] {
+    auto launch = [&](auto kernel) {
+      GKR_LAUNCH(c, kernel, dim3(grid), dim3(kBlock), 0, sa, sb, n, al, da, db, hi, lo, h, sk, tw);
+    };
+    if (np == 0)
+      launch(k_trip_mfma<KIND, 0>);
+    else if (np == 1)
+      launch(k_trip_mfma<KIND, 1>);
+    else if (np == 2)
+      launch(k_trip_mfma<KIND, 2>);
+    else
+      launch(k_trip_mfma<KIND, 3>);
+  });
 }
 int launch_trip(gkr_ctx* c, int kind, int K, const qm31* sa, const qm31* sb, uint64_t n, int np,
                        const qm31* pend, qm31* da, qm31* db, const qm31* hi, const qm31* lo, int h, int slot,
@@ -292,6 +327,7 @@ int launch_trip(gkr_ctx* c, int kind, int K, const qm31* sa, const qm31* sb, uin
   // split layout of k_trip); long ones one lane per entry; up to
   // kTripMaxBlocks workgroups
   const bool split = kind != 2 && 2 * n <= kTripSplitLanes;
+  const bool mfma = kind == 0 && K == 3 && b_chunks == 0 && n >= kMfmaTripMin && n <= kMfmaTripMaxN;
   unsigned grid = partial_grid(split ? 2 * n : n);
   const unsigned max_blocks = K <= 2 ? kTripMaxBlocksShort : kTripMaxBlocks;
   if (grid > max_blocks) grid = max_blocks;
@@ -299,6 +335,12 @@ int launch_trip(gkr_ctx* c, int kind, int K, const qm31* sa, const qm31* sb, uin
   const int nvec = kind == 2 ? 1 : 2;
   TimedLaunch tl(c, kind == 0 ? K_MM_ROUND : K_EQ3_ROUND,
                  16ull * nvec * ((n << np) + (da ? n : 0)));
+  if (mfma) {
+    const uint64_t x = n >> 3;
+    grid = (unsigned)std::min<uint64_t>(x / kMfmaTripX, kMfmaTripBlocks);
+    grid = (unsigned)std::max<uint64_t>(grid, x / kMfmaTripMaxX);
+    return launch_trip_mfma<0>(c, sa, sb, n, np, al, da, db, hi, lo, h, *sk, grid, w, carry_out, carry_in);
+  }
 #define GKR_TRIP_CASE(KI, KK)                                                                                 \
   if (kind == KI && K == KK)                                                                                  \
     return split ? launch_trip_k<KI, KK, true>(c, sa, sb, n, np, al, da, db, hi, lo, h, *sk, grid, b_rows, b_chunks, w, \
