@@ -678,8 +678,8 @@ constexpr uint64_t kTripHuge = GKR_TRIP_HUGE;
 // Rounds per trip over a vector of n entries: 3 up to kTripBig, 2 up to kTripHuge, then 1.
 static inline int trip_k(uint64_t n) { return n > kTripHuge ? 1 : n > kTripBig ? 2 : 3; }
 // Trips of three rounds over kMfmaTripMin to kMfmaTripMaxN entries run on the
-// matrix cores (trip_mfma.h), whatever their length: product sumchecks plan
-// their trips with product_trip_k.  At 2^16 entries and below k_trip<0, 3> is
+// matrix cores (trip_mfma.h), whatever their length: product and eq-sumchecks
+// plan their trips with product_trip_k.  At 2^16 entries and below k_trip<0, 3> is
 // as fast (a 2^16 sumcheck 181 us with either).
 #ifndef GKR_MFMA_TRIP_MIN
 #define GKR_MFMA_TRIP_MIN (1ull << 17)
@@ -1059,7 +1059,7 @@ int product_sumcheck(gkr_ctx* c, PoseidonChannel& ch, int T, const qm31* in_a, c
                             gkr_qm31* round_polys, gkr_qm31* challenges, gkr_qm31* final_a, gkr_qm31* final_b,
                             const qm31* scale3 = nullptr, const FirstTrip* ft = nullptr);
 // Eq-weighted degree-3 sumcheck sum_x eq(z, x) w(x) d(x) (logup.hip): plan and eq tables,
-int eq3_prepare(gkr_ctx* c, const qm31* z, int nv, Eq3Plan* pl, bool with_split = false);
+int eq3_prepare(gkr_ctx* c, const qm31* z, int nv, Eq3Plan* pl, bool with_split = false, int k0 = 0);
 // one trip,
 int eq3_launch_trip(gkr_ctx* c, const Eq3Plan& pl, size_t j, const qm31* w, const qm31* d, int np,
                            const qm31* pend, qm31* dw, qm31* dd, int slot, RoundSink* sk,

@@ -55,9 +55,10 @@ static int device_table(gkr_ctx* c, uint32_t tag, uint32_t log_size, uint32_t** 
 // read (with_split, also the two halves of eq(z, .), Eq3Plan::split_*): the
 // tables' list for k_eq_parts (its point left to the caller), offsets into
 // S_EQPARTS.  arg->count == 0: no tables.
-static int eq3_plan(int nv, bool with_split, Eq3Plan* pl, EqPartsArg* arg_out, uint32_t* total_out) {
+// k0: rounds of the first trip (0: product_trip_k).
+static int eq3_plan(int nv, bool with_split, int k0, Eq3Plan* pl, EqPartsArg* arg_out, uint32_t* total_out) {
   pl->nv = nv;
-  pl->trips = plan_trips(nv, kHostTailEq3, trip_k(1ull << nv));
+  pl->trips = plan_trips(nv, kHostTailEq3, k0 ? k0 : product_trip_k(1ull << nv), product_trip_k);
   pl->hi_off.clear();
   pl->lo_off.clear();
   pl->h.clear();
@@ -105,10 +106,10 @@ static int launch_eq_parts(gkr_ctx* c, const EqPartsArg& arg, uint32_t total, co
 }
 // Plan an eq-sumcheck over 2^nv entries for claim point z and launch the
 // kernel that builds its eq tables (S_EQPARTS).
-int eq3_prepare(gkr_ctx* c, const qm31* z, int nv, Eq3Plan* pl, bool with_split) {
+int eq3_prepare(gkr_ctx* c, const qm31* z, int nv, Eq3Plan* pl, bool with_split, int k0) {
   EqPartsArg arg;
   uint32_t total;
-  TRY(eq3_plan(nv, with_split, pl, &arg, &total));
+  TRY(eq3_plan(nv, with_split, k0, pl, &arg, &total));
   if (!arg.count) return GKR_OK;
   arg.z = make_point(z, nv);
   Posted ps;
@@ -389,7 +390,7 @@ int prelaunch_activation(gkr_ctx* c, const gkr_matrix* input, uint32_t tag, uint
   Eq3Plan epl;
   EqPartsArg arg;
   uint32_t total;
-  TRY(eq3_plan(nv, prep_trip_k(nv) == 0, &epl, &arg, &total));
+  TRY(eq3_plan(nv, prep_trip_k(nv) == 0, prep_trip_k(nv), &epl, &arg, &total));
   uint8_t* pw;
   TRY(ensureT(c, S_PTWAIT, kPtWaitBytes, &pw));
   Posted pp;  // the point
@@ -542,9 +543,9 @@ int prove_activation(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point, 
     c->point_mb = c->pre.want;  // checked once the prepare sums are in
     EqPartsArg arg;
     uint32_t total;
-    TRY(eq3_plan(nv, prep_trip_k(nv) == 0, &epl, &arg, &total));
+    TRY(eq3_plan(nv, prep_trip_k(nv) == 0, prep_trip_k(nv), &epl, &arg, &total));
   } else {
-    TRY(eq3_prepare(c, cpt.data(), nv, &epl, prep_trip_k(nv) == 0));
+    TRY(eq3_prepare(c, cpt.data(), nv, &epl, prep_trip_k(nv) == 0, prep_trip_k(nv)));
   }
 
   // Fiat-Shamir: LOG tag, type tag, gamma, beta (prover.rs:6451-6454)

@@ -327,7 +327,7 @@ int launch_trip(gkr_ctx* c, int kind, int K, const qm31* sa, const qm31* sb, uin
   // split layout of k_trip); long ones one lane per entry; up to
   // kTripMaxBlocks workgroups
   const bool split = kind != 2 && 2 * n <= kTripSplitLanes;
-  const bool mfma = kind == 0 && K == 3 && b_chunks == 0 && n >= kMfmaTripMin && n <= kMfmaTripMaxN;
+  const bool mfma = kind != 2 && K == 3 && b_chunks == 0 && n >= kMfmaTripMin && n <= kMfmaTripMaxN;
   unsigned grid = partial_grid(split ? 2 * n : n);
   const unsigned max_blocks = K <= 2 ? kTripMaxBlocksShort : kTripMaxBlocks;
   if (grid > max_blocks) grid = max_blocks;
@@ -339,7 +339,8 @@ int launch_trip(gkr_ctx* c, int kind, int K, const qm31* sa, const qm31* sb, uin
     const uint64_t x = n >> 3;
     grid = (unsigned)std::min<uint64_t>(x / kMfmaTripX, kMfmaTripBlocks);
     grid = (unsigned)std::max<uint64_t>(grid, x / kMfmaTripMaxX);
-    return launch_trip_mfma<0>(c, sa, sb, n, np, al, da, db, hi, lo, h, *sk, grid, w, carry_out, carry_in);
+    return kind == 0 ? launch_trip_mfma<0>(c, sa, sb, n, np, al, da, db, hi, lo, h, *sk, grid, w, carry_out, carry_in)
+                     : launch_trip_mfma<1>(c, sa, sb, n, np, al, da, db, hi, lo, h, *sk, grid, w, carry_out, carry_in);
   }
 #define GKR_TRIP_CASE(KI, KK)                                                                                 \
   if (kind == KI && K == KK)                                                                                  \

@@ -28,7 +28,7 @@
 // lane l's 16 bytes in slot l: row l % 32 = 16 (c % 2) + 4 word + digit, x
 // block l / 32.  A writing instruction has one (word, digit) for all lanes, so
 // the slot's low four bits are XORed with the lane's (x block, c % 4): 16
-// lanes groups then cover the 64 banks once; the reading lanes permute within
+// groups of four lanes then cover the 64 banks once; the reading lanes permute within
 // the block.  The K order inside a block is 4 (x % 16) + x / 16, the same on
 // both sides.
 //
@@ -39,7 +39,10 @@
 // 7174 -> 4070 us, 2^24 735 -> 508, 2^20 266 -> 244, 2^17 202 -> 192.  Tried:
 // cached loads (4.33 ms), four values folded together (4.16), three waves per
 // SIMD (spills, 4.50), 256 or 1024 workgroups, contiguous or XCD-local ranges
-// per workgroup (no faster).
+// per workgroup (no faster).  Eq-sumchecks take the two factors of their
+// weight one on each side: the Mul layer of 64 x 13824 (2^20 entries, four
+// trips instead of five) 330 -> 309 us, two RMSNorm layers of 64 x 5120 (2^19;
+// Part 0 and Part 1) 2204 -> 2164 us.
 #pragma once
 #include "kernels.h"
 
@@ -192,15 +195,11 @@ static __global__ void __launch_bounds__(kBlock, 2) k_trip_mfma(const qm31* __re
         for (int i = 0; i < 4; i++) st_q(dst, pos + 16 * i, v[i]);
       }
     }
-    if constexpr (KIND == 1) {
-      if (side == 0) {
-        const uint64_t mask = (1ull << eq_h) - 1;
+    if constexpr (KIND == 1) {  // eq(x) = hi * lo, one factor on each side
+      const uint64_t mask = (1ull << eq_h) - 1;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const uint64_t x = x0 + 16 * i;
-          v[i] = qm31_mul(v[i], qm31_mul(ld_q(eq_hi, x >> eq_h), ld_q(eq_lo, x & mask)));
-        }
-      }
+      for (int i = 0; i < 4; i++)
+        v[i] = qm31_mul(v[i], side ? ld_q(eq_lo, (x0 + 16 * i) & mask) : ld_q(eq_hi, (x0 + 16 * i) >> eq_h));
     }
     uint32_t* blk = reinterpret_cast<uint32_t*>(buf[p][side][c >> 1][xl >> 3]) + (xl & 3);
 #pragma unroll

@@ -46,3 +46,17 @@ def test_without_launches_ahead(monkeypatch, logn):
     assert ctx.sumcheck_product_noalloc(va.device_ptr, vb.device_ptr, n, G.PoseidonChannel()) == \
         O.sumcheck_product(a, b, O.Channel())
     ctx.close()
+
+
+@pytest.mark.parametrize("logn", [16, 17, 18, 19])
+@pytest.mark.parametrize("what", ["edges", "same", "uniform"])
+def test_eq_weighted_trips(gpu_ctx, logn, what):
+    """The Mul layer's eq-sumcheck over full QM31 operands."""
+    n = 1 << logn
+    a, b = vec(n, what, logn), vec(n, what, logn + 50)
+    gch, och = G.PoseidonChannel(), O.Channel()
+    pt = gch.draw_qm31s(logn)
+    assert pt == och.draw_qm31s(logn)
+    v = (1, 2, 3, 4)
+    assert gpu_ctx.reduce_mul_layer(pt, v, a, b, gch) == O.reduce_mul_layer(pt, v, a, b, och)
+    assert gch.digest() == och.digest()
