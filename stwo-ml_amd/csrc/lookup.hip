@@ -41,10 +41,9 @@ struct LkRound {
   const qm31* src_den;
   qm31* dst_num;
   qm31* dst_den;
-  qm31 x;         // pending fold challenge
   uint32_t fmt;   // numerator format of the source
   uint32_t gp;    // grand product: den holds the column
-  uint32_t pend;  // fold the source (2^(m+1) entries) with x first
+  uint32_t pend;  // fold the source (2^(m+1) entries) with the last round's challenge first
   uint32_t m;     // variables of the vector summed
   uint32_t wg0;   // first workgroup
   uint32_t slot;  // result slot
@@ -64,22 +63,15 @@ __device__ __forceinline__ qm31 lk_num(const void* p, uint32_t fmt, uint64_t i) 
   return qm31_one();
 }
 
+// The last descriptor whose first workgroup is at most this one (descriptors
+// in workgroup order): every thread tests some at once, one memory round trip
+// (a binary search by one thread took one per step, about 5 us of 96).
 template <typename T>
 __device__ __forceinline__ uint32_t find_desc(const T* d, uint32_t n) {
-  __shared__ uint32_t s_idx;
-  if (threadIdx.x == 0) {
-    uint32_t lo = 0, hi = n - 1;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi + 1) >> 1;
-      if (d[mid].wg0 <= blockIdx.x)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    s_idx = lo;
-  }
-  __syncthreads();
-  return s_idx;
+  uint32_t below = 0;
+  for (uint32_t i = 0; i < n; i += blockDim.x)
+    below += (uint32_t)__syncthreads_count(i + threadIdx.x < n && d[i + threadIdx.x].wg0 <= blockIdx.x);
+  return below - 1;
 }
 
 // One launch: per instance, `levels` circuit levels below level src_log.
@@ -168,10 +160,33 @@ __device__ __forceinline__ qm31 fold_num(const void* p, uint32_t fmt, uint64_t i
   return qm31_fold(a, lk_num(p, fmt, i + h), x);
 }
 
-static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __restrict__ desc, uint32_t n_desc,
+// Where a round's results go: `out` in coherent host memory (kLkRes slots per
+// instance).  A workgroup writes its instance's slots from wave 0 and counts
+// itself on `counter` (a system-scope acquire-release count, after the
+// writes); the last of gridDim.x, when it reaches base + gridDim.x, publishes
+// `seq`.
+struct LkSink {
+  qm31* out;
+  uint32_t* counter;
+  uint32_t base;
+  uint32_t* flag;
+  uint32_t seq;
+};
+__device__ __forceinline__ void lk_publish(const LkSink& sk) {  // every lane of wave 0, after its writes
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+  if (threadIdx.x == 0) {
+    const uint32_t old = __hip_atomic_fetch_add(sk.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (old == sk.base + gridDim.x - 1) publish_flag(sk.flag, sk.seq);
+  }
+}
+
+// x: the last round's challenge, for the instances with a pending fold.
+// direct: every instance has one workgroup, whose sums go to the sink at once
+// (else to partials, for k_lk_finish).
+static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __restrict__ desc, uint32_t n_desc, qm31 x,
                                                              const qm31* __restrict__ tab, const qm31* __restrict__ y,
                                                              int n_y, qm31* __restrict__ partials,
-                                                             qm31* __restrict__ res) {
+                                                             qm31* __restrict__ res, LkSink sk, uint32_t direct) {
   const LkRound D = desc[find_desc(desc, n_desc)];
   const int s = (int)D.m - 2;
   const uint64_t nt = 1ull << s;
@@ -186,10 +201,10 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
     const uint64_t pos[4] = {2 * j, 2 * j + 1, 2 * (nt + j), 2 * (nt + j) + 1};
     qm31 dv[4], nv[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) dv[q] = fold_ld(D.src_den, pos[q], h, pend, D.x);
+    for (int q = 0; q < 4; q++) dv[q] = fold_ld(D.src_den, pos[q], h, pend, x);
     if (!D.gp) {
 #pragma unroll
-      for (int q = 0; q < 4; q++) nv[q] = fold_num(D.src_num, D.fmt, pos[q], h, pend, D.x);
+      for (int q = 0; q < 4; q++) nv[q] = fold_num(D.src_num, D.fmt, pos[q], h, pend, x);
     }
     if (pend) {
 #pragma unroll
@@ -221,7 +236,7 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
       v[3] = qm31_mul(w, qm31_mul(d20, d21));
     }
     if (nt == 1) {  // the last round of this instance: its four values per column
-      qm31* o = res + (uint64_t)kLkRes * D.slot + 4;
+      qm31* o = (direct ? sk.out : res) + (uint64_t)kLkRes * D.slot + 4;
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         o[q] = D.gp ? qm31_zero() : nv[q];
@@ -229,13 +244,23 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
       }
     }
   }
-  block_sum_store<4>(v, partials + 4ull * blockIdx.x);
+  if (!direct) {
+    block_sum_store<4>(v, partials + 4ull * blockIdx.x);
+    return;
+  }
+  __shared__ qm31 sums[4];
+  block_sum_store<4>(v, sums);
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  if (threadIdx.x < 4) sk.out[(uint64_t)kLkRes * D.slot + threadIdx.x] = sums[threadIdx.x];
+  lk_publish(sk);
 }
 
-// Per instance (one workgroup each): the sum of its workgroup rows.
+// Per instance (one workgroup each): the sum of its workgroup rows and, in its
+// last round, its values, delivered to the sink.
 static __global__ void __launch_bounds__(kBlock) k_lk_finish(const LkRound* __restrict__ desc,
                                                               const qm31* __restrict__ partials,
-                                                              qm31* __restrict__ res) {
+                                                              const qm31* __restrict__ res, LkSink sk) {
   const LkRound D = desc[blockIdx.x];
   const uint64_t nt = 1ull << (D.m - 2);
   const uint32_t nwg = (uint32_t)((nt + kBlock - 1) / kBlock);
@@ -248,7 +273,16 @@ static __global__ void __launch_bounds__(kBlock) k_lk_finish(const LkRound* __re
   qm31 tot[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) tot[q] = acc[q].reduce();
-  block_sum_store<4>(tot, res + (uint64_t)kLkRes * D.slot);
+  __shared__ qm31 sums[4];
+  block_sum_store<4>(tot, sums);
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  qm31* o = sk.out + (uint64_t)kLkRes * D.slot;
+  if (threadIdx.x < 4)
+    o[threadIdx.x] = sums[threadIdx.x];
+  else if (threadIdx.x < (unsigned)kLkRes && nt == 1)
+    o[threadIdx.x] = ld_q(res, (uint64_t)kLkRes * D.slot + threadIdx.x);
+  lk_publish(sk);
 }
 
 // ------------------------------------------------------------------ host side
@@ -347,6 +381,7 @@ struct Inst {
   }
 };
 
+// (coherent: the result slots kernels write directly)
 int ensure_host(gkr_ctx* c, int hs, size_t bytes, void** out) {
   if (c->hcap[hs] < bytes) {
     if (c->hbuf[hs]) {
@@ -356,7 +391,7 @@ int ensure_host(gkr_ctx* c, int hs, size_t bytes, void** out) {
     c->hbuf[hs] = nullptr;
     c->hcap[hs] = 0;
     const size_t want = bytes < 4096 ? 4096 : bytes;
-    HIP_TRY(hipHostMalloc(&c->hbuf[hs], want, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc(&c->hbuf[hs], want, hs == H_LKRES ? hipHostMallocCoherent : hipHostMallocDefault));
     c->hcap[hs] = want;
   }
   *out = c->hbuf[hs];
@@ -568,7 +603,7 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
     // per active instance: layer variables lv, oracle variables k = lv - 1
     std::vector<size_t> act;
     std::vector<int> lv(ni, 0);
-    std::vector<qm31> sc(ni), corr(ni, qm31_one()), pend_x(ni);
+    std::vector<qm31> sc(ni), corr(ni, qm31_one());
     std::vector<Poly> polys(ni);
     for (size_t i = 0; i < ni; i++)
       if (I[i].active) {
@@ -581,12 +616,19 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
     if (layer > 0) TRY(lk_tables(c, ood, &d_tab, &d_y));
     std::vector<qm31> assign(layer);
     std::vector<qm31> snap(ni * 8);
+    // every round's instances (those in their own rounds) and launch
+    // descriptors, uploaded once per layer: only the challenge changes
+    struct LayerRound {
+      size_t first, n;
+      uint32_t wg;
+      uint64_t bytes;
+    };
+    std::vector<LkRound> desc;
+    std::vector<size_t> real_all;
+    std::vector<LayerRound> rounds;
+    uint32_t max_wg = 0;
     for (int r = 0; r < layer; r++) {
-      // the instances in their own rounds, and their launch descriptors
-      std::vector<LkRound> d;
-      std::vector<size_t> real;
-      uint32_t wg = 0;
-      uint64_t bytes = 0;
+      LayerRound lr{desc.size(), 0, 0, 0};
       for (size_t i : act) {
         const int k = lv[i] - 1;
         if (layer - r > k) continue;
@@ -615,50 +657,66 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
           e.dst_num = x.fold_num[b];
           e.dst_den = x.fold_den[b];
           e.pend = 1;
-          e.x = pend_x[i];
         }
         e.gp = x.gp();
         e.m = (uint32_t)(lv[i] - rho);
-        e.wg0 = wg;
-        e.slot = (uint32_t)real.size();
+        e.wg0 = lr.wg;
+        e.slot = (uint32_t)lr.n++;
         const uint64_t nt = 1ull << (e.m - 2);
-        wg += (uint32_t)((nt + kBlock - 1) / kBlock);
+        lr.wg += (uint32_t)((nt + kBlock - 1) / kBlock);
         const uint64_t ent = 4 * nt, per_num = e.fmt == NF_Q ? 16 : e.fmt == NF_M31 ? 4 : 0;
-        bytes += (e.pend ? 2 : 1) * ent * (16 + per_num) + (e.pend ? ent * (16 + (fmt_folded == NF_Q ? 16 : 0)) : 0);
-        d.push_back(e);
-        real.push_back(i);
+        lr.bytes += (e.pend ? 2 : 1) * ent * (16 + per_num) + (e.pend ? ent * (16 + (fmt_folded == NF_Q ? 16 : 0)) : 0);
+        desc.push_back(e);
+        real_all.push_back(i);
       }
-      if (!d.empty()) {
-        qm31 *part, *res;
-        void *dv, *h, *hr;
-        TRY(ensure(c, S_LKDESC, d.size() * sizeof(LkRound), &dv));
-        LkRound* dd = static_cast<LkRound*>(dv);
-        TRY(ensureT(c, S_LKPART, 4ull * wg, &part));
-        TRY(ensureT(c, S_LKRES, (size_t)kLkRes * d.size(), &res));
-        TRY(ensure_host(c, H_LKDESC, d.size() * sizeof(LkRound), &h));
-        TRY(ensure_host(c, H_LKRES, (size_t)kLkRes * d.size() * sizeof(qm31), &hr));
-        memcpy(h, d.data(), d.size() * sizeof(LkRound));
+      max_wg = std::max(max_wg, lr.wg);
+      rounds.push_back(lr);
+    }
+    LkRound* d_desc = nullptr;
+    qm31 *part = nullptr, *res = nullptr, *hres = nullptr;
+    if (!desc.empty()) {
+      void *dv, *h, *hr;
+      TRY(ensure(c, S_LKDESC, desc.size() * sizeof(LkRound), &dv));
+      d_desc = static_cast<LkRound*>(dv);
+      TRY(ensureT(c, S_LKPART, 4ull * max_wg, &part));
+      TRY(ensureT(c, S_LKRES, (size_t)kLkRes * act.size(), &res));
+      TRY(ensure_host(c, H_LKDESC, desc.size() * sizeof(LkRound), &h));
+      TRY(ensure_host(c, H_LKRES, (size_t)kLkRes * ni * sizeof(qm31), &hr));
+      hres = static_cast<qm31*>(hr);
+      memcpy(h, desc.data(), desc.size() * sizeof(LkRound));
+      HIP_TRY(hipMemcpyAsync(d_desc, h, desc.size() * sizeof(LkRound), hipMemcpyHostToDevice, c->stream));
+    }
+    qm31 last_x = qm31_zero();
+    for (int r = 0; r < layer; r++) {
+      const LayerRound& lr = rounds[r];
+      const LkRound* d = desc.data() + lr.first;
+      const size_t* real = real_all.data() + lr.first;
+      if (lr.n) {
+        LkSink sk;
+        sk.out = hres;
+        sk.flag = c->h_flag;
+        sk.seq = alloc_seq(&c->seq, 1);
+        TRY(arrival_counter(c, (unsigned)lr.n, &sk.counter, &sk.base));
+        const uint32_t direct = lr.wg == lr.n;  // one workgroup per instance: no finisher launch
         {
           HostTimer ht(c, K_HOST_LAUNCH);
-          HIP_TRY(hipMemcpyAsync(dd, h, d.size() * sizeof(LkRound), hipMemcpyHostToDevice, c->stream));
           {
-            TimedLaunch tl(c, K_LOOKUP, bytes);
-            GKR_LAUNCH(c, k_lk_round, dim3(wg), dim3(kBlock), 0, dd, (uint32_t)d.size(), d_tab, d_y,
-                               layer, part, res);
+            TimedLaunch tl(c, K_LOOKUP, lr.bytes);
+            GKR_LAUNCH(c, k_lk_round, dim3(lr.wg), dim3(kBlock), 0, d_desc + lr.first, (uint32_t)lr.n, last_x, d_tab,
+                       d_y, layer, part, res, sk, direct);
           }
           TRY(check_launch(c));
-          GKR_LAUNCH(c, k_lk_finish, dim3((unsigned)d.size()), dim3(kBlock), 0, dd, part, res);
+          if (!direct)
+            GKR_LAUNCH(c, k_lk_finish, dim3((unsigned)lr.n), dim3(kBlock), 0, d_desc + lr.first, part, res, sk);
           TRY(check_launch(c));
-          HIP_TRY(hipMemcpyAsync(hr, res, (size_t)kLkRes * d.size() * sizeof(qm31), hipMemcpyDeviceToHost,
-                                 c->stream));
         }
-        {
-          HostTimer ht(c, K_HOST_WAIT);
-          TRY(sync(c));
+        if (const int rc = wait_result<0>(c, sk.seq, nullptr, K_HOST_WAIT)) {
+          c->trip_count_valid = false;  // how many workgroups counted themselves is unknown
+          return rc;
         }
-        const qm31* rv = static_cast<const qm31*>(hr);
+        const qm31* rv = hres;
         RootInv roots[kLkMaxVars + 2];
-        for (size_t a = 0; a < real.size(); a++) {
+        for (size_t a = 0; a < lr.n; a++) {
           const size_t i = real[a];
           const qm31* s = rv + (size_t)kLkRes * a;
           const qm31 S0 = I[i].gp() ? s[0] : qm31_add(s[0], qm31_mul(lambda, s[1]));
@@ -702,11 +760,11 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
       round++;
       assign[r] = xr;
       for (size_t i : act) sc[i] = polys[i].eval(xr);
-      for (size_t a = 0; a < real.size(); a++) {
+      for (size_t a = 0; a < lr.n; a++) {
         const size_t i = real[a];
         corr[i] = qm31_mul(corr[i], eq1(xr, ood[layer - (int)d[a].m + 1]));
-        pend_x[i] = xr;
       }
+      last_x = xr;
     }
     // masks: an instance with rounds folds its last four values with the last
     // challenge; a newly joined one gives its level-1 values
