@@ -185,8 +185,9 @@ struct gkr_qvec {
   uint64_t n;
 };
 
-// Pinned host staging buffers (grow-only, hipHostMalloc).
-enum HostSlot { H_LKDESC, H_LKRES, H_LKTAB, H_NSLOTS };
+// Pinned host staging buffers (grow-only, hipHostMalloc; coherent: H_LKRES and
+// H_NORM, which kernels write directly).
+enum HostSlot { H_LKDESC, H_LKRES, H_LKTAB, H_NORM, H_NSLOTS };
 
 // Coherent pinned buffers for the LogUp multiplicities, one per activation
 // layer in flight: a layer's table pass writes its slot, and the layer's proof
@@ -459,6 +460,8 @@ inline uint32_t alloc_seq(uint32_t* counter, uint32_t n) {
 // later.  The partial rows are shared: each finisher consumes them before the
 // next reducing kernel on the stream overwrites them.
 int make_sink(gkr_ctx* c, RoundSink* sk, int slot = 0);
+// Host buffer `hs` (HostSlot) of at least `bytes`.
+int ensure_host(gkr_ctx* c, int hs, size_t bytes, void** out);
 // Launch the one-workgroup finisher that adds `nblocks` partial rows and
 // delivers the NQ results (after a multi-workgroup reducing kernel).
 template <int NQ>
@@ -1077,6 +1080,12 @@ int eq3_sumcheck(gkr_ctx* c, PoseidonChannel& C, const qm31* z, const Eq3Plan& p
 int prove_norm(gkr_ctx* c, bool ln, const gkr_qm31* claim_point, uint32_t n_point, const gkr_qm31* claim_value,
                const gkr_matrix* X, uint64_t dim, const uint32_t* gamma, uint64_t ng, gkr_channel* ch,
                gkr_proof* proof, gkr_norm_out* out, bool commit_gamma);
+// A walk's norm step: the scale as a resident 1 x n matrix (or null); fresh:
+// the claim value is the output's MLE at the point, mixed and returned in
+// *claim_value, from the same device pass as the proof.
+int walk_norm(gkr_ctx* c, bool ln, bool fresh, const gkr_qm31* claim_point, uint32_t n_point, gkr_qm31* claim_value,
+              const gkr_matrix* X, uint64_t dim, const gkr_matrix* gamma, gkr_channel* ch, gkr_proof* proof,
+              gkr_norm_out* out);
 // prove_mle_opening_with_commitment (crypto/mle_opening.rs:1654-1915) over
 // a weight's column-major padded MLE (b) or a resident QM31 vector (q, qn
 // entries, a power of two) (commit.hip); the record gets the claim first when

@@ -24,7 +24,8 @@ namespace {
 constexpr int kLkLevels = 9;   // circuit levels per tree launch
 constexpr int kLkTab = 10;     // suffix eq tables up to 2^10 entries come from the host
 constexpr int kLkMaxVars = 28;
-constexpr int kLkRes = 12;     // result QM31 per instance and round: 4 sums, then 4 num + 4 den values
+constexpr int kLkVals = 8;     // an instance's last values: 4 num + 4 den
+constexpr uint32_t kLkCountedMax = 128;  // workgroups of a round that delivers in its own kernel (20 ns of counting each)
 
 enum : uint32_t { NF_NONE = 0, NF_Q = 1, NF_M31 = 2, NF_ONE = 3 };  // numerator formats
 
@@ -41,12 +42,18 @@ struct LkRound {
   const qm31* src_den;
   qm31* dst_num;
   qm31* dst_den;
+  qm31 weight;    // the instance's power of alpha in the combination
   uint32_t fmt;   // numerator format of the source
   uint32_t gp;    // grand product: den holds the column
   uint32_t pend;  // fold the source (2^(m+1) entries) with the last round's challenge first
   uint32_t m;     // variables of the vector summed
   uint32_t wg0;   // first workgroup
-  uint32_t slot;  // result slot
+  uint32_t slot;  // the instance's slot for its last values
+};
+// Instances of one size: their workgroups are consecutive and their sums are
+// added up.
+struct LkGroup {
+  uint32_t wg0, wg1;  // workgroups [wg0, wg1)
 };
 
 struct LkTop {
@@ -160,33 +167,16 @@ __device__ __forceinline__ qm31 fold_num(const void* p, uint32_t fmt, uint64_t i
   return qm31_fold(a, lk_num(p, fmt, i + h), x);
 }
 
-// Where a round's results go: `out` in coherent host memory (kLkRes slots per
-// instance).  A workgroup writes its instance's slots from wave 0 and counts
-// itself on `counter` (a system-scope acquire-release count, after the
-// writes); the last of gridDim.x, when it reaches base + gridDim.x, publishes
-// `seq`.
-struct LkSink {
-  qm31* out;
-  uint32_t* counter;
-  uint32_t base;
-  uint32_t* flag;
-  uint32_t seq;
-};
-__device__ __forceinline__ void lk_publish(const LkSink& sk) {  // every lane of wave 0, after its writes
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-  if (threadIdx.x == 0) {
-    const uint32_t old = __hip_atomic_fetch_add(sk.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (old == sk.base + gridDim.x - 1) publish_flag(sk.flag, sk.seq);
-  }
-}
-
-// x: the last round's challenge, for the instances with a pending fold.
-// direct: every instance has one workgroup, whose sums go to the sink at once
-// (else to partials, for k_lk_finish).
+// x: the last round's challenge, for the instances with a pending fold.  A
+// workgroup's two sums (t = 0, 2) are weight * (numerators + lambda *
+// denominators), so a size's instances need no sums of their own.
+// counter: one size on at most kLkCountedMax workgroups, the last of which to
+// arrive (the counter reaches base + gridDim.x) adds the rows and delivers
+// them; null: k_lk_finish does.
 static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __restrict__ desc, uint32_t n_desc, qm31 x,
                                                              const qm31* __restrict__ tab, const qm31* __restrict__ y,
-                                                             int n_y, qm31* __restrict__ partials,
-                                                             qm31* __restrict__ res, LkSink sk, uint32_t direct) {
+                                                             int n_y, qm31 lambda, qm31* __restrict__ vals,
+                                                             RoundSink sk, uint32_t* counter, uint32_t base) {
   const LkRound D = desc[find_desc(desc, n_desc)];
   const int s = (int)D.m - 2;
   const uint64_t nt = 1ull << s;
@@ -194,7 +184,7 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
   __shared__ qm31 s_hi;
   if (s > kLkTab && threadIdx.x == 0) s_hi = lk_hi(y, n_y, s, j >> kLkTab);
   __syncthreads();
-  qm31 v[4] = {qm31_zero(), qm31_zero(), qm31_zero(), qm31_zero()};
+  qm31 v[2] = {qm31_zero(), qm31_zero()};
   if (j < nt) {
     const uint64_t h = 1ull << D.m;  // fold distance in the source
     const bool pend = D.pend != 0;
@@ -219,7 +209,7 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
     const qm31 d20 = qm31_sub(qm31_add(dv[2], dv[2]), dv[0]), d21 = qm31_sub(qm31_add(dv[3], dv[3]), dv[1]);
     if (D.gp) {
       v[0] = qm31_mul(w, qm31_mul(dv[0], dv[1]));
-      v[2] = qm31_mul(w, qm31_mul(d20, d21));
+      v[1] = qm31_mul(w, qm31_mul(d20, d21));
     } else {
       qm31 num0, num2;
       if (D.fmt == NF_ONE) {
@@ -230,13 +220,11 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
         num0 = qm31_add(qm31_mul(nv[0], dv[1]), qm31_mul(nv[1], dv[0]));
         num2 = qm31_add(qm31_mul(n20, d21), qm31_mul(n21, d20));
       }
-      v[0] = qm31_mul(w, num0);
-      v[1] = qm31_mul(w, qm31_mul(dv[0], dv[1]));
-      v[2] = qm31_mul(w, num2);
-      v[3] = qm31_mul(w, qm31_mul(d20, d21));
+      v[0] = qm31_mul(w, qm31_add(num0, qm31_mul(lambda, qm31_mul(dv[0], dv[1]))));
+      v[1] = qm31_mul(w, qm31_add(num2, qm31_mul(lambda, qm31_mul(d20, d21))));
     }
     if (nt == 1) {  // the last round of this instance: its four values per column
-      qm31* o = (direct ? sk.out : res) + (uint64_t)kLkRes * D.slot + 4;
+      qm31* o = vals + (uint64_t)kLkVals * D.slot;
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         o[q] = D.gp ? qm31_zero() : nv[q];
@@ -244,45 +232,77 @@ static __global__ void __launch_bounds__(kBlock) k_lk_round(const LkRound* __res
       }
     }
   }
-  if (!direct) {
-    block_sum_store<4>(v, partials + 4ull * blockIdx.x);
+  __shared__ qm31 row[2];
+  block_sum_store<2>(v, row);
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  if (!counter) {
+    if (lane < 2) st_q(sk.partials, 2ull * blockIdx.x + lane, qm31_mul(D.weight, row[lane]));
     return;
   }
-  __shared__ qm31 sums[4];
-  block_sum_store<4>(v, sums);
-  __syncthreads();
-  if (threadIdx.x >= 64) return;
-  if (threadIdx.x < 4) sk.out[(uint64_t)kLkRes * D.slot + threadIdx.x] = sums[threadIdx.x];
-  lk_publish(sk);
+  // The rows travel in device-scope stores and loads, which bypass the XCDs'
+  // caches: this wave's row is in memory once its stores have completed, so
+  // the count needs no release of its own (a release writes back the folded
+  // vectors this kernel left in the L2, about 10 us a round).
+  if (lane < 2) st_q_dev(sk.partials + 2ull * blockIdx.x + lane, qm31_mul(D.weight, row[lane]));
+  wait_memory();
+  uint32_t old = 0;
+  if (lane == 0) old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  old = (uint32_t)__shfl((int)old, 0, 64);
+  if (old != base + gridDim.x - 1) return;
+  wait_memory();
+  qacc acc[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    acc[q].zero();
+    for (uint32_t b = lane; b < gridDim.x; b += 64) acc[q].add(ld_q_dev(sk.partials + 2ull * b + q));
+  }
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const qm31 t = wave_sum(acc[q].reduce());
+    if (lane == 0) sk.out[q] = t;
+  }
+  if (lane == 0) publish_flag(sk.flag, sk.seq);
 }
 
-// Per instance (one workgroup each): the sum of its workgroup rows and, in its
-// last round, its values, delivered to the sink.
-static __global__ void __launch_bounds__(kBlock) k_lk_finish(const LkRound* __restrict__ desc,
-                                                              const qm31* __restrict__ partials,
-                                                              const qm31* __restrict__ res, LkSink sk) {
-  const LkRound D = desc[blockIdx.x];
-  const uint64_t nt = 1ull << (D.m - 2);
-  const uint32_t nwg = (uint32_t)((nt + kBlock - 1) / kBlock);
-  qacc acc[4];
+// Per size (one workgroup each): the sum of its workgroup rows; then, in the
+// last round, the instances' values (n_vals QM31).  All of it goes to
+// coherent host memory (sums at sk.out, values at host_vals); every workgroup
+// writes from wave 0 and counts itself on `counter` (a system-scope
+// acquire-release count), and the last, when it reaches base + gridDim.x,
+// publishes.
+constexpr int kLkFinishBlock = 1024;
+static __global__ void __launch_bounds__(kLkFinishBlock) k_lk_finish(const LkGroup* __restrict__ groups, RoundSink sk,
+                                                                     const qm31* __restrict__ vals, uint32_t n_vals,
+                                                                     qm31* __restrict__ host_vals, uint32_t* counter,
+                                                                     uint32_t base) {
+  const LkGroup g = groups[blockIdx.x];
+  qacc acc[2];
+  acc[0].zero();
+  acc[1].zero();
+  for (uint32_t b = g.wg0 + threadIdx.x; b < g.wg1; b += blockDim.x)
 #pragma unroll
-  for (int q = 0; q < 4; q++) acc[q].zero();
-  for (uint32_t b = threadIdx.x; b < nwg; b += blockDim.x)
+    for (int q = 0; q < 2; q++) acc[q].add(ld_q(sk.partials, 2ull * b + q));
+  __shared__ qm31 sh[kLkFinishBlock / 64][2];
 #pragma unroll
-    for (int q = 0; q < 4; q++) acc[q].add(ld_q(partials, 4ull * (D.wg0 + b) + q));
-  qm31 tot[4];
-#pragma unroll
-  for (int q = 0; q < 4; q++) tot[q] = acc[q].reduce();
-  __shared__ qm31 sums[4];
-  block_sum_store<4>(tot, sums);
+  for (int q = 0; q < 2; q++) {
+    const qm31 t = wave_sum(acc[q].reduce());
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][q] = t;
+  }
   __syncthreads();
   if (threadIdx.x >= 64) return;
-  qm31* o = sk.out + (uint64_t)kLkRes * D.slot;
-  if (threadIdx.x < 4)
-    o[threadIdx.x] = sums[threadIdx.x];
-  else if (threadIdx.x < (unsigned)kLkRes && nt == 1)
-    o[threadIdx.x] = ld_q(res, (uint64_t)kLkRes * D.slot + threadIdx.x);
-  lk_publish(sk);
+  if (threadIdx.x < 2) {
+    qm31 t = sh[0][threadIdx.x];
+    for (int w = 1; w < kLkFinishBlock / 64; w++) t = qm31_add(t, sh[w][threadIdx.x]);
+    sk.out[2 * blockIdx.x + threadIdx.x] = t;
+  }
+  for (uint32_t i = blockIdx.x * 64 + threadIdx.x; i < n_vals; i += gridDim.x * 64) host_vals[i] = ld_q(vals, i);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+  if (threadIdx.x == 0) {
+    const uint32_t old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (old == base + gridDim.x - 1) publish_flag(sk.flag, sk.seq);
+  }
 }
 
 // ------------------------------------------------------------------ host side
@@ -380,23 +400,6 @@ struct Inst {
     }
   }
 };
-
-// (coherent: the result slots kernels write directly)
-int ensure_host(gkr_ctx* c, int hs, size_t bytes, void** out) {
-  if (c->hcap[hs] < bytes) {
-    if (c->hbuf[hs]) {
-      HIP_TRY(hipStreamSynchronize(c->stream));
-      (void)hipHostFree(c->hbuf[hs]);
-    }
-    c->hbuf[hs] = nullptr;
-    c->hcap[hs] = 0;
-    const size_t want = bytes < 4096 ? 4096 : bytes;
-    HIP_TRY(hipHostMalloc(&c->hbuf[hs], want, hs == H_LKRES ? hipHostMallocCoherent : hipHostMallocDefault));
-    c->hcap[hs] = want;
-  }
-  *out = c->hbuf[hs];
-  return GKR_OK;
-}
 
 int lk_check(const gkr_lookup_instance* in, size_t n) {
   if (!in || n == 0) return fail(GKR_ERR_INVALID, "empty lookup batch");
@@ -600,153 +603,181 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
         if (I[i].active) C.mix_felts_stwo(I[i].claims, I[i].nclaims);
     }
     const qm31 alpha = C.draw_qm31(), lambda = C.draw_qm31();
-    // per active instance: layer variables lv, oracle variables k = lv - 1
+    // per active instance: layer variables lv.  The round polynomials are only
+    // needed in the combination sum_a alpha^a r_a (a: position among the active
+    // instances), and a round's polynomial is linear in the instance's sums and
+    // claim with factors that depend on its size alone: so the combination is
+    // formed per size, from the device's alpha-weighted sums and the weighted
+    // claims.
     std::vector<size_t> act;
     std::vector<int> lv(ni, 0);
-    std::vector<qm31> sc(ni), corr(ni, qm31_one());
-    std::vector<Poly> polys(ni);
-    for (size_t i = 0; i < ni; i++)
-      if (I[i].active) {
-        act.push_back(i);
-        lv[i] = layer - (n_layers - (int)I[i].nv) + 1;
-        sc[i] = horner(I[i].claims, I[i].nclaims, lambda);
-        sc[i] = qm31_mul_m31(sc[i], 1u << (layer - (lv[i] - 1)));  // claim doubling for unused variables
-      }
+    std::vector<qm31> power(ni);
+    struct Size {
+      int lv;
+      qm31 sc;    // sum of alpha^a times the claim (doubled for unused variables)
+      qm31 corr;  // eq factors of the rounds done
+      Poly poly;
+    };
+    std::vector<Size> sizes;  // by increasing lv
+    {
+      std::map<int, qm31> claim_of;
+      qm31 pw = qm31_one();
+      for (size_t i = 0; i < ni; i++)
+        if (I[i].active) {
+          act.push_back(i);
+          lv[i] = layer - (n_layers - (int)I[i].nv) + 1;
+          const qm31 sc = qm31_mul_m31(horner(I[i].claims, I[i].nclaims, lambda), 1u << (layer - (lv[i] - 1)));
+          power[i] = pw;
+          const auto at = claim_of.emplace(lv[i], qm31_zero()).first;
+          at->second = qm31_add(at->second, qm31_mul(pw, sc));
+          pw = qm31_mul(pw, alpha);
+        }
+      for (const auto& e : claim_of) sizes.push_back(Size{e.first, e.second, qm31_one(), Poly()});
+    }
     qm31 *d_tab = nullptr, *d_y = nullptr;
     if (layer > 0) TRY(lk_tables(c, ood, &d_tab, &d_y));
     std::vector<qm31> assign(layer);
-    std::vector<qm31> snap(ni * 8);
-    // every round's instances (those in their own rounds) and launch
+    // every round's instances (those in their own rounds, by size) and launch
     // descriptors, uploaded once per layer: only the challenge changes
     struct LayerRound {
-      size_t first, n;
+      size_t first, n;      // descriptors
+      size_t gfirst, ng;    // groups; their sizes are sizes[s0 ..]
+      size_t s0;
       uint32_t wg;
       uint64_t bytes;
     };
     std::vector<LkRound> desc;
-    std::vector<size_t> real_all;
+    std::vector<LkGroup> groups;
     std::vector<LayerRound> rounds;
     uint32_t max_wg = 0;
     for (int r = 0; r < layer; r++) {
-      LayerRound lr{desc.size(), 0, 0, 0};
-      for (size_t i : act) {
-        const int k = lv[i] - 1;
-        if (layer - r > k) continue;
-        const int rho = r - (layer - k);
-        const Inst& x = I[i];
-        LkRound e;
-        memset(&e, 0, sizeof e);
-        const void* n0;
-        const qm31* d0;
-        uint32_t fmt0;
-        x.layer(lv[i], &n0, &d0, &fmt0);
-        const uint32_t fmt_folded = fmt0 == NF_ONE ? NF_ONE : x.gp() ? NF_NONE : NF_Q;
-        // own round rho reads the layer (rho <= 1) or the buffer round rho - 1
-        // wrote, and (rho >= 1) folds into buffer (rho - 1) & 1
-        if (rho <= 1) {
-          e.src_num = n0;
-          e.src_den = d0;
-          e.fmt = fmt0;
-        } else {
-          e.src_num = x.fold_num[rho & 1];
-          e.src_den = x.fold_den[rho & 1];
-          e.fmt = fmt_folded;
+      LayerRound lr{desc.size(), 0, groups.size(), 0, 0, 0, 0};
+      for (size_t si = 0; si < sizes.size(); si++) {
+        const int k = sizes[si].lv - 1;
+        if (layer - r > k) {  // a constant round of smaller instances (the first sizes)
+          lr.s0 = si + 1;
+          continue;
         }
-        if (rho >= 1) {
-          const int b = (rho - 1) & 1;
-          e.dst_num = x.fold_num[b];
-          e.dst_den = x.fold_den[b];
-          e.pend = 1;
+        const uint32_t wg_begin = lr.wg;
+        for (size_t a = 0; a < act.size(); a++) {
+          const size_t i = act[a];
+          if (lv[i] != sizes[si].lv) continue;
+          const int rho = r - (layer - k);
+          const Inst& x = I[i];
+          LkRound e;
+          memset(&e, 0, sizeof e);
+          const void* n0;
+          const qm31* d0;
+          uint32_t fmt0;
+          x.layer(lv[i], &n0, &d0, &fmt0);
+          const uint32_t fmt_folded = fmt0 == NF_ONE ? NF_ONE : x.gp() ? NF_NONE : NF_Q;
+          // own round rho reads the layer (rho <= 1) or the buffer round rho - 1
+          // wrote, and (rho >= 1) folds into buffer (rho - 1) & 1
+          if (rho <= 1) {
+            e.src_num = n0;
+            e.src_den = d0;
+            e.fmt = fmt0;
+          } else {
+            e.src_num = x.fold_num[rho & 1];
+            e.src_den = x.fold_den[rho & 1];
+            e.fmt = fmt_folded;
+          }
+          if (rho >= 1) {
+            const int b = (rho - 1) & 1;
+            e.dst_num = x.fold_num[b];
+            e.dst_den = x.fold_den[b];
+            e.pend = 1;
+          }
+          e.weight = power[i];
+          e.gp = x.gp();
+          e.m = (uint32_t)(lv[i] - rho);
+          e.wg0 = lr.wg;
+          e.slot = (uint32_t)a;
+          const uint64_t nt = 1ull << (e.m - 2);
+          lr.wg += (uint32_t)((nt + kBlock - 1) / kBlock);
+          const uint64_t ent = 4 * nt, per_num = e.fmt == NF_Q ? 16 : e.fmt == NF_M31 ? 4 : 0;
+          lr.bytes += (e.pend ? 2 : 1) * ent * (16 + per_num) + (e.pend ? ent * (16 + (fmt_folded == NF_Q ? 16 : 0)) : 0);
+          desc.push_back(e);
+          lr.n++;
         }
-        e.gp = x.gp();
-        e.m = (uint32_t)(lv[i] - rho);
-        e.wg0 = lr.wg;
-        e.slot = (uint32_t)lr.n++;
-        const uint64_t nt = 1ull << (e.m - 2);
-        lr.wg += (uint32_t)((nt + kBlock - 1) / kBlock);
-        const uint64_t ent = 4 * nt, per_num = e.fmt == NF_Q ? 16 : e.fmt == NF_M31 ? 4 : 0;
-        lr.bytes += (e.pend ? 2 : 1) * ent * (16 + per_num) + (e.pend ? ent * (16 + (fmt_folded == NF_Q ? 16 : 0)) : 0);
-        desc.push_back(e);
-        real_all.push_back(i);
+        groups.push_back(LkGroup{wg_begin, lr.wg});
+        lr.ng++;
       }
       max_wg = std::max(max_wg, lr.wg);
       rounds.push_back(lr);
     }
     LkRound* d_desc = nullptr;
-    qm31 *part = nullptr, *res = nullptr, *hres = nullptr;
+    LkGroup* d_groups = nullptr;
+    qm31 *part = nullptr, *vals = nullptr, *hres = nullptr, *hvals = nullptr;
     if (!desc.empty()) {
+      const size_t db = desc.size() * sizeof(LkRound), gb = groups.size() * sizeof(LkGroup);
       void *dv, *h, *hr;
-      TRY(ensure(c, S_LKDESC, desc.size() * sizeof(LkRound), &dv));
+      TRY(ensure(c, S_LKDESC, db + gb, &dv));
       d_desc = static_cast<LkRound*>(dv);
-      TRY(ensureT(c, S_LKPART, 4ull * max_wg, &part));
-      TRY(ensureT(c, S_LKRES, (size_t)kLkRes * act.size(), &res));
-      TRY(ensure_host(c, H_LKDESC, desc.size() * sizeof(LkRound), &h));
-      TRY(ensure_host(c, H_LKRES, (size_t)kLkRes * ni * sizeof(qm31), &hr));
+      d_groups = reinterpret_cast<LkGroup*>(static_cast<uint8_t*>(dv) + db);
+      TRY(ensureT(c, S_LKPART, 2ull * max_wg, &part));
+      TRY(ensureT(c, S_LKRES, (size_t)kLkVals * act.size(), &vals));
+      TRY(ensure_host(c, H_LKDESC, db + gb, &h));
+      TRY(ensure_host(c, H_LKRES, (2 * (size_t)kLkMaxVars + (size_t)kLkVals * ni) * sizeof(qm31), &hr));
       hres = static_cast<qm31*>(hr);
-      memcpy(h, desc.data(), desc.size() * sizeof(LkRound));
-      HIP_TRY(hipMemcpyAsync(d_desc, h, desc.size() * sizeof(LkRound), hipMemcpyHostToDevice, c->stream));
+      hvals = hres + 2 * kLkMaxVars;
+      memcpy(h, desc.data(), db);
+      memcpy(static_cast<uint8_t*>(h) + db, groups.data(), gb);
+      HIP_TRY(hipMemcpyAsync(dv, h, db + gb, hipMemcpyHostToDevice, c->stream));
     }
     qm31 last_x = qm31_zero();
     for (int r = 0; r < layer; r++) {
       const LayerRound& lr = rounds[r];
-      const LkRound* d = desc.data() + lr.first;
-      const size_t* real = real_all.data() + lr.first;
+      const bool last = r + 1 == layer;  // every size's last round: the instances' values too
       if (lr.n) {
-        LkSink sk;
+        RoundSink sk;
+        sk.partials = part;
         sk.out = hres;
         sk.flag = c->h_flag;
         sk.seq = alloc_seq(&c->seq, 1);
-        TRY(arrival_counter(c, (unsigned)lr.n, &sk.counter, &sk.base));
-        const uint32_t direct = lr.wg == lr.n;  // one workgroup per instance: no finisher launch
+        const bool counted = !last && lr.ng == 1 && lr.wg <= kLkCountedMax;
+        uint32_t* counter = nullptr;
+        uint32_t base = 0;
+        TRY(arrival_counter(c, counted ? lr.wg : (unsigned)lr.ng, &counter, &base));
         {
           HostTimer ht(c, K_HOST_LAUNCH);
           {
             TimedLaunch tl(c, K_LOOKUP, lr.bytes);
             GKR_LAUNCH(c, k_lk_round, dim3(lr.wg), dim3(kBlock), 0, d_desc + lr.first, (uint32_t)lr.n, last_x, d_tab,
-                       d_y, layer, part, res, sk, direct);
+                       d_y, layer, lambda, vals, sk, counted ? counter : nullptr, base);
           }
           TRY(check_launch(c));
-          if (!direct)
-            GKR_LAUNCH(c, k_lk_finish, dim3((unsigned)lr.n), dim3(kBlock), 0, d_desc + lr.first, part, res, sk);
+          if (!counted)
+            GKR_LAUNCH(c, k_lk_finish, dim3((unsigned)lr.ng), dim3(kLkFinishBlock), 0, d_groups + lr.gfirst, sk, vals,
+                       last ? (uint32_t)(kLkVals * act.size()) : 0u, hvals, counter, base);
           TRY(check_launch(c));
         }
         if (const int rc = wait_result<0>(c, sk.seq, nullptr, K_HOST_WAIT)) {
           c->trip_count_valid = false;  // how many workgroups counted themselves is unknown
           return rc;
         }
-        const qm31* rv = hres;
-        RootInv roots[kLkMaxVars + 2];
-        for (size_t a = 0; a < lr.n; a++) {
-          const size_t i = real[a];
-          const qm31* s = rv + (size_t)kLkRes * a;
-          const qm31 S0 = I[i].gp() ? s[0] : qm31_add(s[0], qm31_mul(lambda, s[1]));
-          const qm31 S2 = I[i].gp() ? s[2] : qm31_add(s[2], qm31_mul(lambda, s[3]));
-          const int m = (int)d[a].m;
-          const qm31 yc = ood[layer - m + 1];
-          const qm31 r0 = qm31_mul(qm31_mul(S0, corr[i]), eq1(qm31_zero(), yc));
-          const qm31 r2 = qm31_mul(qm31_mul(S2, corr[i]), eq1(two, yc));
-          if (!roots[m].valid) roots[m] = root_inv(yc);
-          polys[i] = cubic_with_root(r0, qm31_sub(sc[i], r0), r2, roots[m]);
-          if (m == 2)
-            for (int q = 0; q < 8; q++) snap[8 * i + q] = s[4 + q];
-        }
       }
       Poly comb;
-      for (size_t a = act.size(); a-- > 0;) {
-        const size_t i = act[a];
-        const int k = lv[i] - 1;
-        if (layer - r > k) {  // a constant round of a smaller instance
-          polys[i].c[0] = qm31_mul(sc[i], inv2);
-          polys[i].len = 1;
-          polys[i].trunc();
+      for (size_t si = 0; si < sizes.size(); si++) {
+        Size& z = sizes[si];
+        if (si < lr.s0) {  // a constant round
+          z.poly = Poly();
+          z.poly.c[0] = qm31_mul(z.sc, inv2);
+          z.poly.len = 1;
+          z.poly.trunc();
+        } else {
+          const qm31* s = hres + 2 * (si - lr.s0);
+          const qm31 yc = ood[layer - (z.lv - (r - (layer - (z.lv - 1)))) + 1];
+          const qm31 r0 = qm31_mul(qm31_mul(s[0], z.corr), eq1(qm31_zero(), yc));
+          const qm31 r2 = qm31_mul(qm31_mul(s[1], z.corr), eq1(two, yc));
+          z.poly = cubic_with_root(r0, qm31_sub(z.sc, r0), r2, root_inv(yc));
         }
-        if (!qm31_eq(qm31_add(polys[i].eval(qm31_zero()), polys[i].eval(qm31_one())), sc[i]))
+        if (!qm31_eq(qm31_add(z.poly.eval(qm31_zero()), z.poly.eval(qm31_one())), z.sc))
           return fail(GKR_ERR_INVALID, "lookup batch: round %d of layer %d does not sum to the claim (degenerate input)",
                       r, layer);
-        for (int q = 0; q < comb.len; q++) comb.c[q] = qm31_mul(comb.c[q], alpha);
-        const int len = std::max(comb.len, polys[i].len);
+        const int len = std::max(comb.len, z.poly.len);
         for (int q = 0; q < len; q++)
-          comb.c[q] = qm31_add(q < comb.len ? comb.c[q] : qm31_zero(), q < polys[i].len ? polys[i].c[q] : qm31_zero());
+          comb.c[q] = qm31_add(q < comb.len ? comb.c[q] : qm31_zero(), q < z.poly.len ? z.poly.c[q] : qm31_zero());
         comb.len = len;
       }
       qm31 xr;
@@ -759,10 +790,10 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
       out->round_poly_lens[round] = (uint32_t)comb.len;
       round++;
       assign[r] = xr;
-      for (size_t i : act) sc[i] = polys[i].eval(xr);
-      for (size_t a = 0; a < lr.n; a++) {
-        const size_t i = real[a];
-        corr[i] = qm31_mul(corr[i], eq1(xr, ood[layer - (int)d[a].m + 1]));
+      for (size_t si = 0; si < sizes.size(); si++) {
+        Size& z = sizes[si];
+        z.sc = z.poly.eval(xr);
+        if (si >= lr.s0) z.corr = qm31_mul(z.corr, eq1(xr, ood[layer - (z.lv - (r - (layer - (z.lv - 1)))) + 1]));
       }
       last_x = xr;
     }
@@ -771,7 +802,8 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
     std::vector<qm31> mk(4 * ni);
     {
       HostTimer ht(c, K_HOST_FS);
-      for (size_t i : act) {
+      for (size_t a = 0; a < act.size(); a++) {
+        const size_t i = act[a];
         const Inst& x = I[i];
         qm31* m = &mk[4 * i];
         if (lv[i] == 1) {
@@ -780,7 +812,7 @@ extern "C" int gkr_prove_lookup_batch(gkr_ctx* c, gkr_channel* ch, const gkr_loo
           m[2] = x.top[4];
           m[3] = x.top[5];
         } else {
-          const qm31* s = &snap[8 * i];
+          const qm31* s = hvals + kLkVals * a;
           const qm31 xl = assign[layer - 1];
           const qm31 n0 = qm31_fold(s[0], s[2], xl), n1 = qm31_fold(s[1], s[3], xl);
           const qm31 d0 = qm31_fold(s[4], s[6], xl), d1 = qm31_fold(s[5], s[7], xl);

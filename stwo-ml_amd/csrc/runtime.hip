@@ -193,6 +193,22 @@ int dot2_evals(gkr_ctx* c, const qm31* z, int nv, const uint32_t* v0, const uint
   TRY(dot2_launch(c, z, nv, v0, v1, 0, &sk));
   return wait_sink<2>(c, sk, out);
 }
+int ensure_host(gkr_ctx* c, int hs, size_t bytes, void** out) {
+  if (c->hcap[hs] < bytes) {
+    if (c->hbuf[hs]) {
+      HIP_TRY(hipStreamSynchronize(c->stream));
+      (void)hipHostFree(c->hbuf[hs]);
+    }
+    c->hbuf[hs] = nullptr;
+    c->hcap[hs] = 0;
+    const size_t want = bytes < 4096 ? 4096 : bytes;
+    HIP_TRY(hipHostMalloc(&c->hbuf[hs], want,
+                          hs == H_LKRES || hs == H_NORM ? hipHostMallocCoherent : hipHostMallocDefault));
+    c->hcap[hs] = want;
+  }
+  *out = c->hbuf[hs];
+  return GKR_OK;
+}
 int make_sink(gkr_ctx* c, RoundSink* sk, int slot) {
   qm31* part;
   TRY(ensureT(c, S_PART, (size_t)kMaxSums * kMaxPartialBlocks, &part));
