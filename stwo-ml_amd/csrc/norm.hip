@@ -17,24 +17,73 @@
 #include "internal.h"
 #include "norm.h"
 
+#include <algorithm>
+
 // ------------------------------------------------------------------ kernels
-// Per real row r (one workgroup each): sums mod P of x and x^2 over the first
-// `active` columns (S1, S2) and over all columns (T1, T2), to out[4r .. 4r+3].
-static __global__ void __launch_bounds__(kBlock) k_norm_rows(const uint32_t* __restrict__ X, uint64_t cols,
-                                                            uint64_t active, uint32_t* __restrict__ out) {
-  const uint32_t* row = X + (uint64_t)blockIdx.x * cols;
+// norm_rsqrt of a table key (below 2^16): the float square root is within one
+// of the integer one there.
+__device__ __forceinline__ uint32_t rsqrt_entry(uint32_t v) {
+  uint32_t s = (uint32_t)sqrtf((float)v);
+  while (s * s > v) s--;
+  while ((s + 1) * (s + 1) <= v) s++;
+  return s == 0 ? (1u << 16) - 1 : (1u << 16) / s;
+}
+// A row's statistics from its sums S1 = sum x, S2 = sum x^2 over the active
+// columns (act = active mod P, inv_n its inverse): LayerNorm mean = S1 /
+// active and key = variance = (S2 - 2 mean S1 + active mean^2) / active,
+// RMSNorm key = rms^2 = S2 / active; keys masked to the table.  On host and
+// device: the device builds the vectors from them without a round trip.
+struct RowStat {
+  uint32_t mean, key;
+};
+GKR_HD RowStat row_stat(bool layernorm, uint32_t s1, uint32_t s2, uint32_t act, uint32_t inv_n) {
+  if (!layernorm) return RowStat{0u, m31_mul(s2, inv_n) & kNormMask};
+  const uint32_t mean = m31_mul(s1, inv_n);
+  const uint32_t vs =
+      m31_add(m31_sub(s2, m31_mul(m31_add(mean, mean), s1)), m31_mul(act, m31_mul(mean, mean)));
+  return RowStat{mean, m31_mul(vs, inv_n) & kNormMask};
+}
+
+// Per padded row r (one workgroup each): sums mod P of x and x^2 over the
+// first `active` columns (S1, S2) and over all columns (T1, T2), to out[4r ..
+// 4r+3] in host memory; (mean or 0, rsqrt) to rowv[2r .. 2r+1].  Rows past the
+// matrix are zero.  Bound by a row's chain of loads: four in flight per thread,
+// and 1024 threads where a row has work for them; many or short rows take a
+// wave each, which also keeps grids below 2^32 threads.
+constexpr int kNormRowBlock = 1024;
+constexpr uint64_t kNormWideRows = 1ull << 16;
+inline int norm_row_block(uint64_t rows, uint64_t cols) {
+  return cols >= kNormRowBlock && rows <= kNormWideRows ? kNormRowBlock : 64;
+}
+static __global__ void __launch_bounds__(kNormRowBlock) k_norm_rows(const uint32_t* __restrict__ X, uint64_t rows,
+                                                                   uint64_t cols, uint64_t active, int layernorm,
+                                                                   uint32_t act, uint32_t inv_n,
+                                                                   uint32_t* __restrict__ out,
+                                                                   uint32_t* __restrict__ rowv) {
+  const uint64_t r = blockIdx.x;
+  const uint32_t nt = blockDim.x;
+  const uint32_t* row = X + r * cols;
   uint64_t s1 = 0, s2 = 0, t1 = 0, t2 = 0;
-  for (uint64_t c = threadIdx.x; c < cols; c += blockDim.x) {
-    const uint32_t x = row[c];
-    const uint32_t x2 = m31_mul(x, x);
-    t1 += x;
-    t2 += x2;
-    if (c < active) {
-      s1 += x;
-      s2 += x2;
+  if (r < rows) {
+    for (uint64_t c0 = threadIdx.x; c0 < cols; c0 += 4 * nt) {
+      uint32_t x[4];  // four loads in flight
+#pragma unroll
+      for (int u = 0; u < 4; u++) x[u] = c0 + u * nt < cols ? row[c0 + u * nt] : 0u;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const uint32_t x2 = m31_mul(x[u], x[u]);
+        t1 += x[u];
+        t2 += x2;
+        if (c0 + u * nt < active) {
+          s1 += x[u];
+          s2 += x2;
+        }
+      }
     }
   }
-  __shared__ uint64_t sh[4][kBlock / 64];
+  constexpr int W = kNormRowBlock / 64;
+  __shared__ uint64_t sh[4][W];
+  __shared__ uint32_t tot[4];
   uint64_t v[4] = {s1, s2, t1, t2};
 #pragma unroll
   for (int q = 0; q < 4; q++) {
@@ -44,8 +93,15 @@ static __global__ void __launch_bounds__(kBlock) k_norm_rows(const uint32_t* __r
   __syncthreads();
   if (threadIdx.x < 4) {
     uint64_t s = 0;
-    for (int w = 0; w < kBlock / 64; w++) s += sh[threadIdx.x][w] % P;
-    out[4 * (uint64_t)blockIdx.x + threadIdx.x] = (uint32_t)(s % P);
+    for (int w = 0; w < (int)(nt / 64); w++) s += sh[threadIdx.x][w] % P;
+    tot[threadIdx.x] = (uint32_t)(s % P);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *reinterpret_cast<uint4*>(out + 4 * r) = make_uint4(tot[0], tot[1], tot[2], tot[3]);
+    const RowStat st = row_stat(layernorm != 0, tot[0], tot[1], act, inv_n);
+    rowv[2 * r] = st.mean;
+    rowv[2 * r + 1] = rsqrt_entry(st.key);
   }
 }
 
@@ -55,13 +111,16 @@ static __global__ void __launch_bounds__(kBlock) k_norm_rows(const uint32_t* __r
 // in_q = x, out = centered * rsqrt.  RMSNorm: w = x, d = scale = rsqrt *
 // gamma[min(col, ng - 1)] on the active columns (rsqrt elsewhere), out = x *
 // scale on the active columns (x elsewhere); in_q is not written.
+// *bad_gamma (host memory) is set when a gamma value is not canonical.
 static __global__ void k_norm_prepare(const uint32_t* __restrict__ X, uint64_t rows, uint64_t cols, int log_pcol,
                                       uint64_t n, int layernorm, uint64_t active, const uint32_t* __restrict__ rowv,
                                       const uint32_t* __restrict__ gamma, uint64_t ng, qm31* __restrict__ w,
                                       qm31* __restrict__ d, qm31* __restrict__ in_q, uint32_t* __restrict__ in_u,
-                                      uint32_t* __restrict__ out_u) {
+                                      uint32_t* __restrict__ out_u, uint32_t* __restrict__ bad_gamma) {
   const uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
+  for (uint64_t i = p; i < ng; i += n)
+    if (gamma[i] >= P) *bad_gamma = 1;
   const uint64_t r = p >> log_pcol, c = p & ((1ull << log_pcol) - 1);
   const uint32_t x = (r < rows && c < cols) ? X[r * cols + c] : 0u;
   const uint32_t mean = rowv[2 * r], rs = rowv[2 * r + 1];
@@ -111,12 +170,25 @@ std::vector<qm31> as_q(const std::vector<uint32_t>& v) {
   return q;
 }
 
-// Forward statistics of both layers (prover.rs:7968-8020, 8447-8487) from the
-// device row sums: LayerNorm mean = S1 / active, variance = (S2 - 2 mean S1 +
-// active mean^2) / active masked to the table, rsqrt = table[variance];
-// RMSNorm rms^2 = (S2 / active) masked, rsqrt = table[rms^2].  Padding rows
-// are zero.  Also the whole-vector sums Part 0 mixes.
-int norm_stats(gkr_ctx* c, const gkr_matrix* X, bool ln, uint64_t dim, NormShape* S) {
+// The layer's shape and everything its proof needs on the device, in one pass
+// without a host round trip: row sums and statistics (k_norm_rows), the padded
+// vectors S_W0 (w), S_D0 (d), S_E0 (LayerNorm input as QM31), S_MIN (input
+// u32), S_MOUT (output u32) (k_norm_prepare), and the MLEs of input and output
+// at z; then the statistics on the host (prover.rs:7968-8020, 8447-8487): keys,
+// rsqrt values and the whole-vector sums Part 0 mixes.  The scale comes from
+// the host (gamma, ng values) or from device memory (d_gamma).  *bad_gamma: a
+// scale value is not canonical.  (Two RMSNorm layers of 64 x 5120 with fresh
+// claims, against a round trip after the sums and after the vectors, the whole
+// pass run for the claim and again for the proof, and Part 2's host rounds in
+// scalar code: 2200 -> 1575 us.)
+struct NormReady {
+  NormShape S;
+  qm31 input_eval, output_eval;
+  bool bad_gamma = false;
+};
+int norm_setup(gkr_ctx* c, const gkr_matrix* X, bool ln, uint64_t dim, const uint32_t* gamma, uint64_t ng,
+               const uint32_t* d_gamma, const qm31* z, int n_z, NormReady* R) {
+  NormShape* S = &R->S;
   S->ln = ln;
   S->rows = X->rows;
   S->cols = X->cols;
@@ -129,96 +201,76 @@ int norm_stats(gkr_ctx* c, const gkr_matrix* X, bool ln, uint64_t dim, NormShape
   if (S->nv == 0) return fail(GKR_ERR_INVALID, "norm layer over a single entry has no rounds");
   if (dim == 0) return fail(GKR_ERR_INVALID, "norm layer with no active column");
   if (S->nv > kMaxVars) return fail(GKR_ERR_INVALID, "norm layer too large");
-  std::vector<uint32_t> sums(4 * X->rows);
-  uint32_t* d_sums;
-  TRY(ensureT(c, S_NORMSUM, 4 * X->rows, &d_sums));
+  if (n_z != S->nv) return fail(GKR_ERR_INVALID, "point has %d vars, the norm MLE has %d", n_z, S->nv);
+  if (S->n != (1ull << S->nv)) return fail(GKR_ERR_DEVICE, "norm vectors of %llu entries over %d variables",
+                                           (unsigned long long)S->n, S->nv);
+  if (ln) ng = 0;
   const uint64_t act_real = S->active < X->cols ? S->active : X->cols;
-  {
-    TimedLaunch tl(c, K_NORM, 4 * X->rows * X->cols + 16 * X->rows);
-    GKR_LAUNCH(c, k_norm_rows, dim3((unsigned)X->rows), dim3(kBlock), 0, X->dev, X->cols, act_real,
-                       d_sums);
-  }
-  TRY(check_launch(c));
-  HIP_TRY(hipMemcpyAsync(sums.data(), d_sums, sums.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-  TRY(sync(c));
   const uint32_t act_m = m31_from_u32((uint32_t)(S->active % P));
   const uint32_t inv_n = S->active ? m31_inv(act_m) : 0u;
   const uint32_t pcol_m = m31_from_u32((uint32_t)(S->pcol % P));
+  // host side: the row sums, the gamma flag, the scale's staging
+  void* hv;
+  const uint64_t stage = gamma && !d_gamma ? ng : 0;
+  TRY(ensure_host(c, H_NORM, (4 * S->prow + 4 + stage) * sizeof(uint32_t), &hv));
+  uint32_t* sums = static_cast<uint32_t*>(hv);
+  uint32_t* bad = sums + 4 * S->prow;
+  *bad = 0;
+  uint32_t *d_rowv, *in_u, *out_u;
+  qm31 *w, *d, *in_q, *eq_hi, *eq_lo;
+  TRY(ensureT(c, S_NORMROW, 2 * S->prow + stage, &d_rowv));
+  TRY(ensureT(c, S_W0, S->n, &w));
+  TRY(ensureT(c, S_D0, S->n, &d));
+  TRY(ensureT(c, S_E0, ln ? S->n : 1, &in_q));
+  TRY(ensureT(c, S_MIN, S->n, &in_u));
+  TRY(ensureT(c, S_MOUT, S->n, &out_u));
+  TRY(ensureT(c, S_EQHI, 1ull << (S->nv - S->nv / 2), &eq_hi));
+  TRY(ensureT(c, S_EQLO, 1ull << (S->nv / 2), &eq_lo));
+  if (stage) {
+    memcpy(bad + 4, gamma, ng * sizeof(uint32_t));
+    HIP_TRY(hipMemcpyAsync(d_rowv + 2 * S->prow, bad + 4, ng * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
+    d_gamma = d_rowv + 2 * S->prow;
+  }
+  {
+    TimedLaunch tl(c, K_NORM, 4 * X->rows * X->cols + 16 * X->rows);
+    GKR_LAUNCH(c, k_norm_rows, dim3((unsigned)S->prow), dim3(norm_row_block(S->prow, X->cols)), 0, X->dev, X->rows, X->cols, act_real,
+               ln ? 1 : 0, act_m, inv_n, sums, d_rowv);
+  }
+  TRY(check_launch(c));
+  {  // reads X once; writes w, d (and the LayerNorm input) as QM31, input and output as u32
+    TimedLaunch tl(c, K_NORM, 4 * S->rows * S->cols + (ln ? 56 : 40) * S->n);
+    GKR_LAUNCH(c, k_norm_prepare, dim3(grid_for(S->n)), dim3(kBlock), 0, X->dev, S->rows, S->cols,
+               log2_exact(S->pcol), S->n, ln ? 1 : 0, S->active, d_rowv, d_gamma, d_gamma ? ng : 0, w, d, in_q, in_u,
+               out_u, bad);
+  }
+  TRY(check_launch(c));
+  qm31 io[2];
+  TRY(dot2_evals(c, z, S->nv, in_u, out_u, io));  // queued behind the kernels writing the sums and the flag
+  R->input_eval = io[0];
+  R->output_eval = io[1];
+  R->bad_gamma = *reinterpret_cast<volatile uint32_t*>(bad) != 0;
   S->key.assign(S->prow, 0);
   S->var.assign(S->prow, 0);
   S->rsq.assign(S->prow, 0);
   S->mean.assign(S->prow, 0);
   S->t1_total = S->cen_sq_total = S->sq_total = 0;
   for (uint64_t r = 0; r < S->prow; r++) {
-    const bool real = r < X->rows;
-    const uint32_t s1 = real ? sums[4 * r] : 0u, s2 = real ? sums[4 * r + 1] : 0u;
-    const uint32_t t1 = real ? sums[4 * r + 2] : 0u, t2 = real ? sums[4 * r + 3] : 0u;
+    const uint32_t s1 = sums[4 * r], s2 = sums[4 * r + 1], t1 = sums[4 * r + 2], t2 = sums[4 * r + 3];
+    const RowStat st = row_stat(ln, s1, s2, act_m, inv_n);
+    S->key[r] = st.key;
+    S->rsq[r] = norm_rsqrt(st.key);
     if (ln) {
-      const uint32_t mean = m31_mul(s1, inv_n);
-      // sum over the active columns of (x - mean)^2 = S2 - 2 mean S1 + active mean^2
-      const uint32_t m2 = m31_mul(mean, mean);
-      const uint32_t vs = m31_add(m31_sub(s2, m31_mul(m31_add(mean, mean), s1)), m31_mul(act_m, m2));
-      const uint32_t var = m31_mul(vs, inv_n) & kNormMask;
-      S->mean[r] = mean;
-      S->var[r] = var;
-      S->key[r] = var;
-      S->rsq[r] = norm_rsqrt(var);
+      S->mean[r] = st.mean;
+      S->var[r] = st.key;
       // Part 0 totals over the whole padded row: sum x and sum (x - mean)^2 over pcol entries
       S->t1_total = m31_add(S->t1_total, t1);
-      const uint32_t row_sq = m31_add(m31_sub(t2, m31_mul(m31_add(mean, mean), t1)), m31_mul(pcol_m, m2));
+      const uint32_t row_sq = m31_add(m31_sub(t2, m31_mul(m31_add(st.mean, st.mean), t1)),
+                                      m31_mul(pcol_m, m31_mul(st.mean, st.mean)));
       S->cen_sq_total = m31_add(S->cen_sq_total, row_sq);
     } else {
-      const uint32_t ms = m31_mul(s2, inv_n) & kNormMask;
-      S->key[r] = ms;
-      S->rsq[r] = norm_rsqrt(ms);
       S->sq_total = m31_add(S->sq_total, t2);
     }
   }
-  return GKR_OK;
-}
-
-// Builds the padded device vectors: S_W0 (w), S_D0 (d), S_E0 (LayerNorm input
-// as QM31), S_MIN (input u32), S_MOUT (output u32).
-int norm_prepare(gkr_ctx* c, const gkr_matrix* X, const NormShape& S, const uint32_t* gamma, uint64_t ng) {
-  std::vector<uint32_t> rowv(2 * S.prow);
-  for (uint64_t r = 0; r < S.prow; r++) {
-    rowv[2 * r] = S.ln ? S.mean[r] : 0u;
-    rowv[2 * r + 1] = S.rsq[r];
-  }
-  uint32_t *d_rowv, *d_gamma = nullptr, *in_u, *out_u;
-  qm31 *w, *d, *in_q;
-  TRY(ensureT(c, S_NORMROW, rowv.size() + (gamma ? ng : 0), &d_rowv));
-  if (gamma && ng) d_gamma = d_rowv + rowv.size();
-  TRY(ensureT(c, S_W0, S.n, &w));
-  TRY(ensureT(c, S_D0, S.n, &d));
-  TRY(ensureT(c, S_E0, S.ln ? S.n : 1, &in_q));
-  TRY(ensureT(c, S_MIN, S.n, &in_u));
-  TRY(ensureT(c, S_MOUT, S.n, &out_u));
-  HIP_TRY(hipMemcpyAsync(d_rowv, rowv.data(), rowv.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-  if (d_gamma)
-    HIP_TRY(hipMemcpyAsync(d_gamma, gamma, ng * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-  {  // reads X once; writes w, d (and the LayerNorm input) as QM31, input and output as u32
-    TimedLaunch tl(c, K_NORM, 4 * S.rows * S.cols + (S.ln ? 56 : 40) * S.n);
-    GKR_LAUNCH(c, k_norm_prepare, dim3(grid_for(S.n)), dim3(kBlock), 0, X->dev, S.rows, S.cols,
-                       log2_exact(S.pcol), S.n, S.ln ? 1 : 0, S.active, d_rowv, d_gamma, d_gamma ? ng : 0, w, d,
-                       in_q, in_u, out_u);
-  }
-  TRY(check_launch(c));
-  // the host copies of rowv / gamma must outlive the copies
-  return sync(c);
-}
-
-// MLEs of the input (S_MIN) and output (S_MOUT) at z: one eq split, one pass.
-int norm_evals(gkr_ctx* c, const NormShape& S, const qm31* z, qm31* in_eval, qm31* out_eval) {
-  uint32_t *in_u, *out_u;
-  TRY(ensureT(c, S_MIN, S.n, &in_u));
-  TRY(ensureT(c, S_MOUT, S.n, &out_u));
-  if (S.n != (1ull << S.nv)) return fail(GKR_ERR_DEVICE, "norm vectors of %llu entries over %d variables",
-                                         (unsigned long long)S.n, S.nv);
-  qm31 io[2];
-  TRY(dot2_evals(c, z, S.nv, in_u, out_u, io));
-  *in_eval = io[0];
-  *out_eval = io[1];
   return GKR_OK;
 }
 
@@ -340,21 +392,37 @@ int norm_logup(gkr_ctx* c, PoseidonChannel& C, uint64_t type_tag, const NormShap
   C.mix_u64(0x4C4F47ull);  // "LOG"
   C.mix_u64(type_tag);
   const qm31 gamma = C.draw_qm31(), beta = C.draw_qm31();
+  // the keys that occur, in table order, and the reciprocals of their
+  // denominators (a row's denominator is its key's): one inversion in all
+  std::vector<uint32_t> nz(S.key);
+  std::sort(nz.begin(), nz.end());
+  nz.erase(std::unique(nz.begin(), nz.end()), nz.end());
+  std::vector<qm31> dn(nz.size()), wn(nz.size());
+  for (size_t q = 0; q < nz.size(); q++)
+    dn[q] = qm31_sub(qm31_sub(gamma, qm31_from_m31(nz[q])), qm31_mul(beta, qm31_from_m31(norm_rsqrt(nz[q]))));
+  bool zero = false;
+  qm31 run = qm31_one();
+  for (size_t q = 0; q < nz.size(); q++) {
+    wn[q] = run;
+    zero = zero || qm31_is_zero(dn[q]);
+    run = qm31_mul(run, dn[q]);
+  }
+  run = qm31_inv(run);
+  for (size_t q = nz.size(); q-- > 0;) {
+    wn[q] = zero ? qm31_inv(dn[q]) : qm31_mul(run, wn[q]);
+    run = qm31_mul(run, dn[q]);
+  }
   std::vector<qm31> w(S.prow), d(S.prow), e(S.prow);
-  qm31 wsum = qm31_zero();
+  qm31 wsum = qm31_zero(), table_sum = qm31_zero();
   for (uint64_t r = 0; r < S.prow; r++) {
-    d[r] = qm31_sub(qm31_sub(gamma, qm31_from_m31(S.key[r])), qm31_mul(beta, qm31_from_m31(S.rsq[r])));
-    w[r] = qm31_inv(d[r]);
+    const size_t q = std::lower_bound(nz.begin(), nz.end(), S.key[r]) - nz.begin();
+    d[r] = dn[q];
+    w[r] = wn[q];
     wsum = qm31_add(wsum, w[r]);
   }
   const qm31 trace_sum = qm31_mul_m31(wsum, m31_from_u32((uint32_t)(S.pcol % P)));
-  qm31 table_sum = qm31_zero();
-  for (uint32_t j = 0; j < tsize; j++)
-    if (out->multiplicities[j]) {
-      const qm31 dj =
-          qm31_sub(qm31_sub(gamma, qm31_from_m31(j)), qm31_mul(beta, qm31_from_m31(norm_rsqrt(j))));
-      table_sum = qm31_add(table_sum, qm31_mul_m31(qm31_inv(dj), m31_from_u32(out->multiplicities[j])));
-    }
+  for (size_t q = 0; q < nz.size(); q++)
+    table_sum = qm31_add(table_sum, qm31_mul_m31(wn[q], m31_from_u32(out->multiplicities[nz[q]])));
   if (!qm31_eq(trace_sum, table_sum)) return fail(GKR_ERR_LOGUP, "norm rsqrt LogUp sum mismatch");
   C.mix_secure_field(trace_sum);
   out->claimed_sum = G(trace_sum);
@@ -377,17 +445,8 @@ int norm_logup(gkr_ctx* c, PoseidonChannel& C, uint64_t type_tag, const NormShap
   for (int t = 0; t < S.lr; t++) {
     const size_t mid = len / 2;
     qm31 sk[4];
-    for (int k = 0; k < 4; k++) {
-      const qm31 x = qm31_from_m31((uint32_t)k), omx = qm31_sub(qm31_one(), x);
-      qm31 acc = qm31_zero();
-      for (size_t i = 0; i < mid; i++) {
-        const qm31 et = qm31_add(qm31_mul(omx, e[i]), qm31_mul(x, e[mid + i]));
-        const qm31 wt = qm31_add(qm31_mul(omx, w[i]), qm31_mul(x, w[mid + i]));
-        const qm31 dt = qm31_add(qm31_mul(omx, d[i]), qm31_mul(x, d[mid + i]));
-        acc = qm31_add(acc, qm31_mul(qm31_mul(et, wt), dt));
-      }
-      sk[k] = acc;
-    }
+    hostfield::eq3_round(qwords(e.data()), qwords(w.data()), qwords(d.data()), mid,
+                         reinterpret_cast<uint32_t(*)[4]>(sk));
     const qm31 dd1 = qm31_sub(sk[1], sk[0]);
     const qm31 dd2 = qm31_mul(qm31_add(qm31_sub(qm31_sub(sk[2], sk[1]), sk[1]), sk[0]), inv2);
     const qm31 dd3 = qm31_mul(qm31_sub(qm31_sub(sk[3], sk[0]), qm31_mul(three, qm31_sub(sk[2], sk[1]))), inv6);
@@ -396,11 +455,9 @@ int norm_logup(gkr_ctx* c, PoseidonChannel& C, uint64_t type_tag, const NormShap
     for (int k = 0; k < 4; k++) out->logup_round_polys[4 * t + k] = G(cf[k]);
     C.mix_poly_coeffs_deg3(cf[0], cf[1], cf[2], cf[3]);
     s[t] = C.draw_qm31();
-    for (size_t i = 0; i < mid; i++) {
-      e[i] = qm31_fold(e[i], e[i + mid], s[t]);
-      w[i] = qm31_fold(w[i], w[i + mid], s[t]);
-      d[i] = qm31_fold(d[i], d[i + mid], s[t]);
-    }
+    hostfield::fold(qwords(e.data()), mid, qwords(&s[t]));
+    hostfield::fold(qwords(w.data()), mid, qwords(&s[t]));
+    hostfield::fold(qwords(d.data()), mid, qwords(&s[t]));
     len = mid;
   }
   // column rounds: w d constant, p(X) = K eqlin(z_t, X) with K = e w d prod_{earlier} eqlin(z, s)
@@ -419,9 +476,6 @@ int norm_logup(gkr_ctx* c, PoseidonChannel& C, uint64_t type_tag, const NormShap
   out->in_eval = G(row_mle(as_q(S.key), S.lr, s.data()));
   out->out_eval = G(row_mle(as_q(S.rsq), S.lr, s.data()));
   // multiplicity sumcheck over the 2^16 table, from the nonzero entries
-  std::vector<uint32_t> nz;
-  for (uint32_t j = 0; j < tsize; j++)
-    if (out->multiplicities[j]) nz.push_back(j);
   std::vector<qm31> ew(nz.size(), qm31_one());
   qm31 msum = qm31_zero();
   for (uint32_t j : nz) msum = qm31_add(msum, qm31_from_m31(m31_from_u32(out->multiplicities[j])));
@@ -514,26 +568,30 @@ void record_norm(gkr_proof* proof, bool ln, const qm31& claim, const NormShape& 
 }  // namespace
 
 // Both reducers: ln selects LayerNorm (prover.rs:7944-8395) or RMSNorm
-// (8407-8801, with the optional per-column gamma).
-int prove_norm(gkr_ctx* c, bool ln, const gkr_qm31* claim_point, uint32_t n_point, const gkr_qm31* claim_value,
-               const gkr_matrix* X, uint64_t dim, const uint32_t* gamma, uint64_t ng, gkr_channel* ch,
-               gkr_proof* proof, gkr_norm_out* out, bool commit_gamma) {
+// (8407-8801, with the optional per-column gamma, from the host or d_gamma).
+// fresh: the claim is the output's MLE at the point; it is mixed and written
+// to *claim_value.
+static int prove_norm_core(gkr_ctx* c, bool ln, bool fresh, const gkr_qm31* claim_point, uint32_t n_point,
+                           gkr_qm31* claim_value, const gkr_matrix* X, uint64_t dim, const uint32_t* gamma,
+                           uint64_t ng, const uint32_t* d_gamma, gkr_channel* ch, gkr_proof* proof, gkr_norm_out* out,
+                           bool commit_gamma) {
   CH_CHECK(ch);
   std::vector<qm31> z;
   TRY(norm_check(c, claim_point, n_point, claim_value, X, out, &z));
-  if (gamma && ng)
-    for (uint64_t i = 0; i < ng; i++)
-      if (gamma[i] >= P) return fail(GKR_ERR_INVALID, "gamma value %llu not canonical", (unsigned long long)i);
   HIP_TRY(hipSetDevice(c->device));
   c->mm.valid = false;
   TraceScope trace;
   PoseidonChannel& C = ch->ch;
-  NormShape S;
-  TRY(norm_stats(c, X, ln, dim, &S));
-  TRY(norm_prepare(c, X, S, ln ? nullptr : gamma, ln ? 0 : ng));
+  NormReady R;
+  TRY(norm_setup(c, X, ln, dim, gamma, ng, d_gamma, z.data(), (int)z.size(), &R));
+  if (R.bad_gamma) return fail(GKR_ERR_INVALID, "gamma holds a value that is not canonical");
+  const NormShape& S = R.S;
+  const qm31 input_eval = R.input_eval, output_eval = R.output_eval;
+  if (fresh) {
+    *claim_value = G(output_eval);
+    C.mix_secure_field(output_eval);
+  }
   const qm31 claim = Q(*claim_value);
-  qm31 input_eval, output_eval;
-  TRY(norm_evals(c, S, z.data(), &input_eval, &output_eval));
   const qm31 key_eval = row_mle(as_q(S.key), S.lr, z.data());
   const qm31 rsqrt_eval = row_mle(as_q(S.rsq), S.lr, z.data());
   out->input_eval = G(input_eval);
@@ -558,7 +616,7 @@ int prove_norm(gkr_ctx* c, bool ln, const gkr_qm31* claim_point, uint32_t n_poin
     size_t len = e.size();
     for (int k = S.lr; k < S.nv; k++) {
       const size_t h = len / 2;
-      for (size_t i = 0; i < h; i++) e[i] = qm31_fold(e[i], e[i + h], z[k]);
+      hostfield::fold(qwords(e.data()), h, qwords(&z[k]));
       len = h;
     }
     out->gamma_eval = G(e[0]);
@@ -646,6 +704,26 @@ int prove_norm(gkr_ctx* c, bool ln, const gkr_qm31* claim_point, uint32_t n_poin
   return GKR_OK;
 }
 
+int prove_norm(gkr_ctx* c, bool ln, const gkr_qm31* claim_point, uint32_t n_point, const gkr_qm31* claim_value,
+               const gkr_matrix* X, uint64_t dim, const uint32_t* gamma, uint64_t ng, gkr_channel* ch,
+               gkr_proof* proof, gkr_norm_out* out, bool commit_gamma) {
+  if (!claim_value) return fail(GKR_ERR_INVALID, "null argument");
+  if (gamma && ng)
+    for (uint64_t i = 0; i < ng; i++)
+      if (gamma[i] >= P) return fail(GKR_ERR_INVALID, "gamma value %llu not canonical", (unsigned long long)i);
+  gkr_qm31 value = *claim_value;
+  return prove_norm_core(c, ln, false, claim_point, n_point, &value, X, dim, gamma, ng, nullptr, ch, proof, out,
+                         commit_gamma);
+}
+int walk_norm(gkr_ctx* c, bool ln, bool fresh, const gkr_qm31* claim_point, uint32_t n_point, gkr_qm31* claim_value,
+              const gkr_matrix* X, uint64_t dim, const gkr_matrix* gamma, gkr_channel* ch, gkr_proof* proof,
+              gkr_norm_out* out) {
+  if (gamma && gamma->ctx != c) return fail(GKR_ERR_INVALID, "matrix belongs to another (or a destroyed) context");
+  if (fresh) *claim_value = G(qm31_zero());
+  return prove_norm_core(c, ln, fresh, claim_point, n_point, claim_value, X, dim, nullptr, gamma ? gamma->cols : 0,
+                         gamma ? gamma->dev : nullptr, ch, proof, out, false);
+}
+
 extern "C" int gkr_prove_layernorm_layer(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point,
                                          const gkr_qm31* claim_value, const gkr_matrix* input, uint64_t dim,
                                          gkr_channel* ch, gkr_proof* proof, gkr_norm_out* out) {
@@ -668,17 +746,14 @@ extern "C" int gkr_norm_output_claim(gkr_ctx* c, uint32_t kind, const gkr_matrix
   const bool ln = kind == GKR_STEP_LAYERNORM;
   HIP_TRY(hipSetDevice(c->device));
   c->mm.valid = false;
-  NormShape S;
-  TRY(norm_stats(c, input, ln, dim, &S));
-  if ((int)n_point != S.nv) return fail(GKR_ERR_INVALID, "point has %u vars, the norm MLE has %d", n_point, S.nv);
   std::vector<qm31> z(n_point);
   for (uint32_t l = 0; l < n_point; l++) {
     if (!canonical_q(point[l])) return fail(GKR_ERR_INVALID, "point not canonical");
     z[l] = Q(point[l]);
   }
-  TRY(norm_prepare(c, input, S, ln ? nullptr : gamma, ln ? 0 : n_gamma));
-  qm31 ie, oe;
-  TRY(norm_evals(c, S, z.data(), &ie, &oe));
+  NormReady R;
+  TRY(norm_setup(c, input, ln, dim, gamma, n_gamma, nullptr, z.data(), (int)n_point, &R));
+  const qm31 oe = R.output_eval;
   *value = G(oe);
   return GKR_OK;
 }
