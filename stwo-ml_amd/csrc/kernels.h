@@ -1950,17 +1950,19 @@ static __global__ void k_pad_q(const uint32_t* __restrict__ X, uint64_t rows, ui
   const uint64_t r = p >> log_pcol, c = p & ((1ull << log_pcol) - 1);
   st_q(out, p, qm31_from_m31((r < rows && c < cols) ? m31_from_u32(X[r * cols + c]) : 0u));
 }
-// out[i] = in[i] lifted to QM31; with host_copy (coherent pinned host memory)
-// the raw values are also written there, and with clear_in the input is
-// zeroed behind the read (a histogram left ready for its next use).
-static __global__ void k_u32_to_q(uint32_t* __restrict__ in, uint64_t n, qm31* __restrict__ out,
-                                  uint32_t* __restrict__ host_copy, int clear_in) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// out[i] = in[i] lifted to QM31.
+static __global__ void k_u32_to_q(const uint32_t* __restrict__ in, uint64_t n, qm31* __restrict__ out) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const uint32_t v = in[i];
-  st_q(out, i, qm31_from_m31(m31_from_u32(v)));
-  if (host_copy) host_copy[i] = v;
-  if (clear_in) in[i] = 0;
+  st_q(out, i, qm31_from_m31(m31_from_u32(in[i])));
+}
+// in to coherent pinned host memory, then zeroed (a histogram left ready for
+// its next use).
+static __global__ void k_u32_to_host(uint32_t* __restrict__ in, uint64_t n, uint32_t* __restrict__ host_copy) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  host_copy[i] = in[i];
+  in[i] = 0;
 }
 
 // ------------------------------------------------------------------ MLE evaluation helpers

@@ -604,6 +604,19 @@ int prove_activation(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point, 
   uint32_t* hist = nullptr;
   if (lds_hist) TRY(ensureT(c, S_LKHIST, hgroups * (kHistBins / 2), &hist));
   const std::vector<Trip> mtrips = plan_trips((int)table_log, kHostTailSum, kTripMaxK);
+  // A large table's multiplicities go to their pinned host copy in two halves
+  // (4 MB for 2^20 entries take 77 us at the link's rate), each queued where
+  // the host draws challenges meanwhile: behind the multiplicity sumcheck's
+  // first trip, while it finishes the eq-sumcheck, and behind that sumcheck's
+  // hand-over.  Softmax over 2560 x 64 with the 2^20 table: 622 us with the
+  // whole copy before the first trip, 576 with halves.
+  const uint64_t mult_half = tsize / 2;
+  auto mult_to_host = [&](int half) -> int {
+    GKR_LAUNCH(c, k_u32_to_host, dim3(grid_for(mult_half)), dim3(kBlock), 0, d_mult + half * mult_half, mult_half,
+               c->h_mult + half * mult_half);
+    if (half) c->mult_zero_entries = tsize;
+    return check_launch(c);
+  };
   bool table_side_done = false;
   std::function<int()> table_side = [&]() -> int {
     table_side_done = true;
@@ -630,13 +643,13 @@ int prove_activation(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point, 
       TRY(deliver_args(c, grid, &counter, &base));
       GKR_LAUNCH(c, k_logup_table_sum, dim3(grid), dim3(kBlock), 0, d_inv, d_mult, tsize, sk_table, counter, base);
       TRY(deliver_finish<1>(c, sk_table, grid, counter));
-      // the multiplicities as QM31 for the sumcheck, and to the pinned host copy
-      GKR_LAUNCH(c, k_u32_to_q, dim3(grid_for(tsize)), dim3(kBlock), 0, d_mult, tsize, m0, c->h_mult, 1);
+      // the multiplicities as QM31 for the sumcheck
+      GKR_LAUNCH(c, k_u32_to_q, dim3(grid_for(tsize)), dim3(kBlock), 0, d_mult, tsize, m0);
       TRY(check_launch(c));
-      c->mult_zero_entries = tsize;
     }
-    return launch_trip(c, 2, mtrips[0].K, m0, nullptr, tsize, 0, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
-                       kSlotMult0, &sk_mult0);
+    TRY(launch_trip(c, 2, mtrips[0].K, m0, nullptr, tsize, 0, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
+                    kSlotMult0, &sk_mult0));
+    return lds_hist ? GKR_OK : mult_to_host(0);
   };
 
   // The trace sum goes into the transcript now; the table-side sum it must
@@ -683,6 +696,7 @@ int prove_activation(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point, 
   bool io_launched = false;
   auto launch_io = [&]() -> int {
     io_launched = true;
+    if (!lds_hist) TRY(mult_to_host(1));
     return dot2_launch(c, chal.data(), nv, d_min, d_mout, kSlotIO, &sk_io);
   };
   out->w_eval = G(w_eval);
@@ -794,12 +808,16 @@ int prove_activation(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point, 
     mfin[0] = V[0];
   }
   trace_point(C, "logup.mult");
-  // the kernels whose results were waited for in the multiplicity sumcheck
-  // were queued after the one writing the multiplicities' pinned copy
-  if (out->multiplicities) memcpy(out->multiplicities, c->h_mult, tsize * sizeof(uint32_t));
   if (!io_launched) TRY(launch_io());
+  // the kernels whose results were waited for in the multiplicity sumcheck
+  // were queued after the one writing the multiplicities' pinned copy (its
+  // first half of a large table), the io pass after the second half
+  const uint64_t early = lds_hist ? tsize : mult_half;
+  if (out->multiplicities) memcpy(out->multiplicities, c->h_mult, early * sizeof(uint32_t));
   qm31 io[2];
   TRY(wait_sink<2>(c, sk_io, io));
+  if (out->multiplicities && early < tsize)
+    memcpy(out->multiplicities + early, c->h_mult + early, (tsize - early) * sizeof(uint32_t));
   const qm31 in_eval = io[0], out_eval = io[1];
   out->in_eval = G(in_eval);
   out->out_eval = G(out_eval);
