@@ -12,7 +12,9 @@
 // Representation rules (all values are representatives, not canonical):
 //   normalized: limbs in [0, 2^29), value below 2^261;
 //   mul/sqr inputs: limbs below 2^30 (the sum of two normalized values is
-//     fine), output normalized with value < p + a*b/R;
+//     fine), output normalized with value < p + a*b/R; their signed forms take
+//     limbs of either sign (a difference of two normalized values), and their
+//     output's top limb has the sign of the value;
 //   the linear layer adds limb-wise and subtracts through kD4, a
 //     representation of 4p whose limbs dominate any normalized subtrahend
 //     below 1.1p (limbs 0-7 at least 2^30 - 2, limb 8 at least 2^21 - 2).
@@ -81,6 +83,9 @@ GKR_HD T in_order(T v) {
 // limb 0 of the result.  The sum of the m's is at most 2^261, so the result is
 // below p + t / 2^261; limb 0 is at most 2^29, the others below 2^29.
 //
+// Digits and carries are the same in two's complement, so limbs of either sign
+// (S) only need the signed mad and the arithmetic shift.
+//
 // Per product 81 (or 45 in a square) + 18 v_mad_u64_u32, 16 shifts and about 20
 // 32-bit operations.  k_merkle_level is bound by VALU issue, most of it the
 // mads.  Against unordered columns with the exact digit 2^29 - (t mod 2^29)
@@ -101,8 +106,14 @@ GKR_HD void column_begin(columns& c) {
   c.p6 = opaque(kP6);
   c.p8 = opaque(kP8);
 }
+// a * b of limbs (S: signed)
+template <bool S>
+GKR_HD uint64_t limb_mul(uint32_t a, uint32_t b) {
+  if constexpr (S) return (uint64_t)((int64_t)(int32_t)a * (int32_t)b);
+  return (uint64_t)a * b;
+}
 // the reduction terms and the digit (or result limb) of column k, after its products
-template <int K>
+template <bool S, int K>
 GKR_HD void column_end(columns& c, fe& r) {
   if constexpr (K >= 6 && K < 15) c.acc = in_order(c.acc + (uint64_t)c.m[K - 6] * c.p6);
   if constexpr (K >= 8) c.acc = in_order(c.acc + (uint64_t)c.m[K - 8] * c.p8);
@@ -110,46 +121,51 @@ GKR_HD void column_end(columns& c, fe& r) {
     c.m[K] = (~(uint32_t)c.acc & kMask) + (K == 0 ? 1u : 0u);
   else
     r.l[K - 9] = ((uint32_t)c.acc & kMask) + (K == 9 ? 1u : 0u);
-  c.acc >>= 29;
+  if constexpr (S)
+    c.acc = (uint64_t)((int64_t)c.acc >> 29);
+  else
+    c.acc >>= 29;
 }
 
-template <int K>
+template <bool S, int K>
 GKR_HD void mul_columns(const fe& a, const fe& b, columns& c, fe& r) {
   constexpr int I0 = K > 8 ? K - 8 : 0;
-  c.acc = in_order(c.acc + (uint64_t)a.l[I0] * b.l[K - I0]);  // the carry is this mad's addend
+  c.acc = in_order(c.acc + limb_mul<S>(a.l[I0], b.l[K - I0]));  // the carry is this mad's addend
 #pragma unroll
-  for (int i = I0 + 1; i <= (K < 8 ? K : 8); i++) c.acc = in_order(c.acc + (uint64_t)a.l[i] * b.l[K - i]);
-  column_end<K>(c, r);
-  if constexpr (K < 16) mul_columns<K + 1>(a, b, c, r);
+  for (int i = I0 + 1; i <= (K < 8 ? K : 8); i++) c.acc = in_order(c.acc + limb_mul<S>(a.l[i], b.l[K - i]));
+  column_end<S, K>(c, r);
+  if constexpr (K < 16) mul_columns<S, K + 1>(a, b, c, r);
 }
 // Inputs: limbs whose pairwise products sum below 2^64 - 2^52 in every column
 // (limbs below 2^30 on both sides with top limbs below 2^29, or a normalized
-// value by limbs below 2^31).
+// value by limbs below 2^31).  S: sums within +-(2^63 - 2^52).
+template <bool S = false>
 GKR_HD void mul(const fe& a, const fe& b, fe& r) {
   columns c;
   fe o;
   column_begin(c);
-  mul_columns<0>(a, b, c, o);
+  mul_columns<S, 0>(a, b, c, o);
   o.l[8] = (uint32_t)c.acc;
   r = o;
 }
 
-template <int K>
+template <bool S, int K>
 GKR_HD void sqr_columns(const fe& a, const fe& d, columns& c, fe& r) {
   constexpr int I0 = K > 8 ? K - 8 : 0;
-  c.acc = in_order(c.acc + (uint64_t)a.l[I0] * (2 * I0 < K ? d.l[K - I0] : a.l[I0]));
+  c.acc = in_order(c.acc + limb_mul<S>(a.l[I0], 2 * I0 < K ? d.l[K - I0] : a.l[I0]));
 #pragma unroll
-  for (int i = I0 + 1; 2 * i < K; i++) c.acc = in_order(c.acc + (uint64_t)a.l[i] * d.l[K - i]);
-  if constexpr (K % 2 == 0 && 2 * I0 < K) c.acc = in_order(c.acc + (uint64_t)a.l[K / 2] * a.l[K / 2]);
-  column_end<K>(c, r);
-  if constexpr (K < 16) sqr_columns<K + 1>(a, d, c, r);
+  for (int i = I0 + 1; 2 * i < K; i++) c.acc = in_order(c.acc + limb_mul<S>(a.l[i], d.l[K - i]));
+  if constexpr (K % 2 == 0 && 2 * I0 < K) c.acc = in_order(c.acc + limb_mul<S>(a.l[K / 2], a.l[K / 2]));
+  column_end<S, K>(c, r);
+  if constexpr (K < 16) sqr_columns<S, K + 1>(a, d, c, r);
 }
 // a^2 with d = 2a limb by limb (off-diagonal products taken once against d).
+template <bool S = false>
 GKR_HD void sqr2(const fe& a, const fe& d, fe& r) {
   columns c;
   fe o;
   column_begin(c);
-  sqr_columns<0>(a, d, c, o);
+  sqr_columns<S, 0>(a, d, c, o);
   o.l[8] = (uint32_t)c.acc;
   r = o;
 }

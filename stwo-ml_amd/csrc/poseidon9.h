@@ -29,8 +29,11 @@ struct hades_consts {
   fe first[4][3];  // rounds 0-3 (round 0, lane 2 unused: see y2_round0)
   fe y2_round0;    // (2 + first[0][2])^3: lane 2 of round 0 when the input lane 2 is 2
   fe partial0;     // constant added to lane 2 before partial round 0
-  fe kd[83];       // partial constant r + 1 plus kD4 (r < 82); kD4 alone for r = 82
-  fe last[4][3];   // rounds 87-90
+  fe kd0;          // partial constant 1 plus kD4, for lane 2 after partial round 0
+  fe u1;           // added to u after partial round 0 (see partial_u)
+  fe ku[83];       // partial round r: added to u (ku[0] unused)
+  uint32_t x6[83]; // partial round r: taken from limb 6 of x (signed; x6[0] unused)
+  fe last[4][3];   // rounds 87-90, round 87 less what u and v still carry
 };
 
 GKR_HD void add(const fe& a, const fe& b, fe& r) {
@@ -63,51 +66,51 @@ GKR_HD void full_round(fe& a, fe& b, fe& c, const K& rc0, const K& rc1, const K&
   full_linear(y0, y1, y2, a, b, c);
 }
 
-// u' = 2(2v + u) + Y folded below 2^252 (1 + 2^-16) and normalized, in one
-// carry pass (u, v normalized and below 2^252 (1 + 2^-16), Y below 1.1p with
-// limb 0 up to 2^29).  The multiple of p to subtract, k = max(h - 1, 0) with
-// h = floor(u' / 2^251) up to the carries still to come, is taken from the
-// top limb before the carries; k p only touches limbs 0, 6 and 8 (k <= 15).
-// The bias 2^29 per limb, returned as 1 from the next limb, keeps every limb
-// non-negative: with it a limb is at most 8 * 2^29 - 6 and the carry into it
-// at most 7.
-GKR_HD void partial_u(const fe& u, const fe& v, const fe& Y, fe& r) {
+// The round constants live in u: it is kept as U = u + g_r, where g_r is the
+// constant that x' = u + g_r - Y needs up to a multiple of 2^174, so x' is one
+// subtraction per limb.  With K_r = g_(r+1) - 2 g_r - 4 g_(r-1),
+//   U' = 4V + 2U + Y + K_r,  V' = U,  x' = U - Y - x6 2^174,
+// and K_r is the third addend of the carry pass's additions: it costs nothing.
+// (Constants added to x, which was normalized: 328 VALU instructions a round
+// instead of 301, seven weights of a Qwen2.5-14B layer 122.0 instead of 117.3 ms.)
+//
+// U' is folded to about [p, 2p) and normalized in the same pass: h p less one p
+// is taken off, h = floor(U' / 2^251) up to the carries still to come, from the
+// top limb before the carries.  h p only touches limbs 0, 6 and 8, and the one
+// p's share of limbs 0 and 6 is part of ku.  Every limb sum has to stay in
+// [0, 2^32): 4V + 2U + Y is at most 7 * 2^29 - 6 and the carry at most 7, so a
+// ku limb is at most 2^29 - 8, and limbs 0 and 6 are at least 16 and 16 kP6
+// (h <= 15).  x6, 0 or +-2^28, is there to move limb 6 into that range.
+// (U, V normalized and below 2^252 (1 + 2^-16), Y above -p/16 and below 1.1p
+// with limb 0 up to 2^29.)
+GKR_HD void partial_u(const fe& u, const fe& v, const fe& Y, const fe& ku, fe& r) {
   uint32_t t[kLimbs];
 #pragma unroll
   for (int k = 0; k < kLimbs; k++) t[k] = in_order((in_order((v.l[k] << 1) + u.l[k]) << 1) + Y.l[k]);  // two v_lshl_add
-  const uint32_t h = t[8] >> 19;
-  const uint32_t q = h > 0 ? h - 1 : 0;
-  t[0] -= q;
-  t[6] -= q * kP6;
-  t[8] -= q << 19;
+  const uint32_t top = t[8] + ku.l[8];
+  const int32_t h = (int32_t)top >> 19;
+  t[0] -= (uint32_t)h;
+  t[6] -= (uint32_t)(h * (int32_t)kP6);
   uint32_t c = 0;
 #pragma unroll
   for (int k = 0; k < 8; k++) {
-    const uint32_t x = t[k] + c + (k == 0 ? (1u << 29) : (1u << 29) - 1u);
+    const uint32_t x = t[k] + ku.l[k] + c;
     r.l[k] = x & kMask;
     c = x >> 29;
   }
-  r.l[8] = t[8] + c - 1u;
+  r.l[8] = ((top & (kP8 - 1u)) | kP8) + c;
 }
-// x' = u + kd - Y, normalized (kd holds 4p in limbs that dominate Y's).
-GKR_HD void partial_x(const fe& u, const fe& kd, const fe& Y, fe& x) {
-  uint32_t c = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const uint32_t t = u.l[k] + kd.l[k] + c - Y.l[k];
-    x.l[k] = t & kMask;
-    c = t >> 29;
-  }
-  x.l[8] = u.l[8] + kd.l[8] + c - Y.l[8];
-}
-// One partial round after the first: (u, v, x) -> (u', u, x'), u' in v.
-GKR_HD void partial_round(const fe& u, fe& v, fe& x, const fe& kd) {
+// One partial round after the first: (u, v, x) -> (u', u, x'), u' in v; x has
+// limbs of either sign, up to 2^29 (limb 6: 2^29 + 2^28) in magnitude, and a
+// value between -1.2p and 7p.
+GKR_HD void partial_round(const fe& u, fe& v, fe& x, const fe& ku, uint32_t x6) {
   fe d, x2, Y;
   twice(x, d);
-  sqr2(x, d, x2);
-  mul(x2, d, Y);
-  partial_u(u, v, Y, v);
-  partial_x(u, kd, Y, x);
+  sqr2<true>(x, d, x2);
+  mul<true>(x2, d, Y);
+  partial_u(u, v, Y, ku, v);
+#pragma unroll
+  for (int k = 0; k < kLimbs; k++) x.l[k] = u.l[k] - Y.l[k] - (k == 6 ? x6 : 0u);
 }
 
 // out = hades([l, r, 2])[0]; l, r normalized, Montgomery, below 8p.
@@ -141,8 +144,8 @@ GKR_HD void hash2(const fe& l, const fe& r, const hades_consts& K, fe& out) {
 #pragma unroll
     for (int k = 0; k < kLimbs; k++) {
       const uint32_t un = u.l[k];
-      u.l[k] = 2u * (un + w.l[k] + y.l[k]);
-      x.l[k] = un + K.kd[0].l[k] - 2u * y.l[k];
+      u.l[k] = 2u * (un + w.l[k] + y.l[k]) + K.u1.l[k];
+      x.l[k] = un + K.kd0.l[k] - 2u * y.l[k];
     }
     normalize(u);
     fold(u);
@@ -150,10 +153,12 @@ GKR_HD void hash2(const fe& l, const fe& r, const hades_consts& K, fe& out) {
   }
 #pragma unroll 1
   for (int r = 1; r < 83; r += 2) {  // the two halves exchange the roles of u and v: no copies
-    partial_round(u, v, x, K.kd[r]);
-    partial_round(v, u, x, K.kd[r + 1]);
+    partial_round(u, v, x, K.ku[r], K.x6[r]);
+    partial_round(v, u, x, K.ku[r + 1], K.x6[r + 1]);
   }
-  c = x;
+#pragma unroll
+  for (int k = 0; k < kLimbs; k++) c.l[k] = x.l[k] + consts::d4(k);
+  normalize(c);
   halve(u);
 #pragma unroll
   for (int k = 0; k < kLimbs; k++) {

@@ -26,13 +26,28 @@ void f9_sqr_limbs(const uint32_t* a, uint32_t* out) {
   f9::sqr(load(a), r);
   store(r, out);
 }
-// (u, v, x) -> (u', u, x') with the round's constant kd[r]
+// signed limbs on either side
+void f9_mul_signed(const uint32_t* a, const uint32_t* b, uint32_t* out) {
+  f9::fe r;
+  f9::mul<true>(load(a), load(b), r);
+  store(r, out);
+}
+void f9_sqr_signed(const uint32_t* a, uint32_t* out) {
+  f9::fe d, r;
+  f9::twice(load(a), d);
+  f9::sqr2<true>(load(a), d, r);
+  store(r, out);
+}
+// (u, v, x) -> (u', u, x') with the constants of round r
 void f9_partial_round(uint32_t* u, uint32_t* v, uint32_t* x, int r) {
   f9::fe U = load(u), V = load(v), X = load(x);
-  f9::partial_round(U, V, X, f9::host_setup().k.kd[r]);
+  f9::partial_round(U, V, X, f9::host_setup().k.ku[r], f9::host_setup().k.x6[r]);
   store(U, v);
   store(V, u);
   store(X, x);
 }
-void f9_kd(int r, uint32_t* out) { store(f9::host_setup().k.kd[r], out); }
+void f9_ku(int r, uint32_t* out) {
+  store(f9::host_setup().k.ku[r], out);
+  out[9] = f9::host_setup().k.x6[r];
+}
 }

@@ -79,6 +79,39 @@ def test_products_random_limbs(f9):
         check_reduced(out, val(b) * val(d))
 
 
+def sval(limbs):
+    return sum(int(x) << (29 * k) for k, x in enumerate(limbs.astype(np.int32)))
+
+
+@pytest.mark.parametrize("x", ["plus", "minus", "mixed", "random"])
+def test_signed_products_at_the_limb_bounds(f9, x):
+    """A difference of two normalized values, limb 6 moved by up to 2^28 more, and its double."""
+    rng = random.Random(10)
+    top = [1 << 29] * 6 + [(1 << 29) + (1 << 28), 1 << 29, (1 << 21) - 1]
+    for _ in range(1 if x in ("plus", "minus") else 200):
+        limbs = [{"plus": 1, "minus": -1, "mixed": rng.choice([-1, 0, 1]), "random": rng.uniform(-1, 1)}[x] * t for t in top]
+        a = np.array([int(t) for t in limbs], dtype=np.int32).view(np.uint32)
+        d = np.array([2 * int(t) for t in limbs], dtype=np.int32).view(np.uint32)
+        sq, out = arr([0] * 9), arr([0] * 9)
+        f9.f9_sqr_signed(ptr(a), ptr(sq))
+        check_reduced(sq, sval(a) ** 2)
+        b = arr([1 << 29] + [M29] * 7 + [(1 << 20) - 1]) if x != "random" else sq
+        f9.f9_mul_signed(ptr(b), ptr(d), ptr(out))
+        t = sval(b) * sval(d)
+        assert (sval(out) * R - t) % PF == 0 and t // R <= sval(out) <= PF + t // R + 1
+        assert int(out[0]) <= 1 << 29 and all(int(v) <= M29 for v in out[1:8])
+
+
+def test_partial_round_constants(f9):
+    """The ranges that keep every 32-bit limb sum of the carry pass in place."""
+    for r in range(1, 83):
+        ku = arr([0] * 10)
+        f9.f9_ku(r, ptr(ku))
+        assert all(int(t) <= (1 << 29) - 8 for t in ku[:8]) and int(ku[8]) < 1 << 20
+        assert int(ku[0]) >= 16 and int(ku[6]) >= 16 * (17 << 18)
+        assert int(ku.astype(np.int32)[9]) in (0, 1 << 28, -(1 << 28))
+
+
 @pytest.mark.parametrize("u", ["top", "ones", "zero", "random"])
 @pytest.mark.parametrize("v", ["top", "ones", "zero", "random"])
 def test_partial_round_at_the_value_bounds(f9, u, v):
@@ -86,16 +119,21 @@ def test_partial_round_at_the_value_bounds(f9, u, v):
     top = (1 << 252) + (1 << 235)  # the bound a folded u keeps
     pick = {"top": lambda: top - 1, "ones": lambda: (1 << 252) - 1, "zero": lambda: 0,
             "random": lambda: rng.randrange(top)}
-    for r in (1, 2, 57, 82):
-        kd = arr([0] * 9)
-        f9.f9_kd(r, ptr(kd))
-        for x in (0, 1, PF, 7 * PF, rng.randrange(7 * PF)):
+    for r in range(1, 83):
+        ku = arr([0] * 10)
+        f9.f9_ku(r, ptr(ku))
+        x6 = int(ku.astype(np.int32)[9]) << 174
+        for x in (0, 1, PF, 3 * PF, -1, -PF, rng.randrange(3 * PF), -rng.randrange(PF)):
             uu, vv = pick[u](), pick[v]()
-            U, V, X = arr(split(uu)), arr(split(vv)), arr(split(x))
+            limbs = split(abs(x))
+            U, V = arr(split(uu)), arr(split(vv))
+            X = np.array([t if x >= 0 else -t for t in limbs], dtype=np.int32).view(np.uint32)
             f9.f9_partial_round(ptr(U), ptr(V), ptr(X), r)
             y2 = 2 * pow(x * pow(R, -1, PF), 3, PF) * R  # 2 x^3 in Montgomery form
             assert val(V) == uu
-            assert (val(U) - 4 * vv - 2 * uu - y2) % PF == 0 and val(U) < top
-            assert (val(X) - uu - val(kd) + y2) % PF == 0 and val(X) < 7 * PF + (1 << 240)
-            for out in (U, X):
-                assert all(int(t) <= M29 for t in out[:8]) and int(out[8]) < 1 << 23
+            fold = (PF - (1 << 251))  # the share of p in ku's limbs 0 and 6
+            assert (val(U) - 4 * vv - 2 * uu - y2 - val(ku[:9]) + fold) % PF == 0 and 0 < val(U) < top
+            assert (sval(X) - uu + x6 + y2) % PF == 0 and -1.2 * PF < sval(X) < 3 * PF
+            assert all(int(t) <= M29 for t in U[:8])
+            assert all(abs(int(t)) <= (1 << 29) + ((1 << 28) if k == 6 else 0)
+                       for k, t in enumerate(X.astype(np.int32)[:8]))
