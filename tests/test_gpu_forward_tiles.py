@@ -44,3 +44,9 @@ def test_one_high_value_takes_the_general_path(ctx):
     a, b = O.synthetic(300, 200, 1, 5), O.synthetic(200, 300, 1, 6)
     a[-1, -1] = 1 << 20
     assert np.array_equal(ctx.matmul_forward(ctx.upload(a), ctx.upload(b)).download(), exact(a, b))
+
+
+def test_four_planes_two_column_tiles_per_wave(ctx):
+    """33 x 129 tiles: enough for two column tiles per wave, the last wave's second one past the edge."""
+    a, b = O.synthetic(1030, 40, 0, 8), O.synthetic(40, 4099, 1, 9)
+    assert np.array_equal(ctx.matmul_forward(ctx.upload(a), ctx.upload(b)).download(), exact(a, b))
