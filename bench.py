@@ -542,7 +542,7 @@ def bench_forward(ctx, args):
                    [(b.rows, b.cols) for _, b in pairs])), "macs_per_step": macs},
         "roofline": {"bound": "hbm", "achieved": round(wbytes / dt / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(wbytes / dt / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "k_gemm_m31 (whole step incl. packing and split reduction)",
+                     "kernel": "k_gemm_int8 (whole step incl. packing and split reduction)",
                      "note": "bytes = the weights' digit plane 0 (int8-range), 1 byte per weight"},
         "u32_weight_equivalent_gbps": round(4 * wbytes / dt / 1e9, 1),
         "outputs_sha256_16": digest, "cpu_baseline": None,

@@ -36,8 +36,8 @@
 // each: half of a tree's hashes become one 36-byte gather.  Entries are tested
 // pair by pair, so any matrix may be given the table: a pair with another
 // value is hashed as before.  Seven weights of a Qwen2.5-14B layer: 242.3 ->
-// 122.0 ms (117.3 with the cheaper partial rounds since); one 5120 x 5120 opening, whose folded layers still hash every
-// node: 62.6 -> 52.0 ms.
+// 122.0 ms (116 with the cheaper partial rounds since); one 5120 x 5120
+// opening, whose folded layers still hash every node: 62.6 -> 52.0 ms.
 #pragma once
 #include <stdint.h>
 
