@@ -35,9 +35,16 @@
 // table of them (2.3 MB, resident in every XCD's 4 MB L2) instead of a hash
 // each: half of a tree's hashes become one 36-byte gather.  Entries are tested
 // pair by pair, so any matrix may be given the table: a pair with another
-// value is hashed as before.  Seven weights of a Qwen2.5-14B layer: 242.3 ->
-// 122.0 ms (116 with the cheaper partial rounds since); one 5120 x 5120
-// opening, whose folded layers still hash every node: 62.6 -> 52.0 ms.
+// value is hashed.  Every lane takes a pair at a time, gathered or hashed: with
+// lanes that took a leaf where others took a pair, a wave's lanes fell out of
+// step and hashed at different iterations.  One commitment of 5120 x 13824 by
+// the share of entries outside [-127, 127], without the table, in single
+// leaves, in pairs: none 81.6, 32.1, 32.1 ms, 0.4% (int8 with -128) 81.6, 63.0,
+// 44.1, 2% 81.6, 87.3, 58.7, 50% 81.6, 165.9, 61.0, all 81.6, 61.4, 61.4 (the
+// times without it are of costlier partial rounds: hashing all is 61.4 now).
+// Seven weights of a Qwen2.5-14B layer: 242.3 -> 122.0 ms (116 with the cheaper
+// partial rounds since); one 5120 x 5120 opening, whose folded layers still
+// hash every node: 62.6 -> 52.0 ms.
 #pragma once
 #include <stdint.h>
 
@@ -194,20 +201,28 @@ static __global__ void __launch_bounds__(kMerkleBlock) k_merkle_level(const Merk
   f9::fe v;
   for (uint32_t r = 0; r < (1u << d); r++) {
     uint32_t lvl = 0, rr = r;
-    bool paired = false;
-    if (T.pairs && !(r & 1)) {  // leaves r, r + 1: rows b, b + 1 of one column, 0 outside the matrix
+    if (T.pairs) {  // leaves r, r + 1: rows b, b + 1 of one column, 0 outside the matrix
       const uint64_t j = (c0 + r) >> T.log_pk, b = (c0 + r) & ((1ull << T.log_pk) - 1);
-      const uint32_t x = pair_side(j < T.cols && b < T.rows ? T.src[b * T.cols + j] : 0u);
-      const uint32_t y = pair_side(j < T.cols && b + 1 < T.rows ? T.src[(b + 1) * T.cols + j] : 0u);
-      paired = x < kPairSide && y < kPairSide;
-      if (paired) {
-        v = T.pairs[x * kPairSide + y];
+      const uint32_t x = j < T.cols && b < T.rows ? T.src[b * T.cols + j] : 0u;
+      const uint32_t y = j < T.cols && b + 1 < T.rows ? T.src[(b + 1) * T.cols + j] : 0u;
+      const uint32_t xi = pair_side(x), yi = pair_side(y);
+      r++;  // whether or not it is in the table: lanes that differ in this stay in step
+      if (xi < kPairSide && yi < kPairSide) {
+        v = T.pairs[xi * kPairSide + yi];
         lvl = 1;
-        rr = r >> 1;
-        r++;
+        rr >>= 1;
+      } else {
+        f9::fe leaf;
+        merkle_leaf_limbs(x, 0, 0, 0, leaf);
+        f9::mul(leaf, C.r2, v);
+        stack[0][threadIdx.x] = v;
+        merkle_leaf_limbs(y, 0, 0, 0, leaf);
+        f9::mul(leaf, C.r2, v);
+        rr = r;
       }
+    } else {
+      merkle_child(T, s, c0 + r, C, v);
     }
-    if (!paired) merkle_child(T, s, c0 + r, C, v);
     while (rr & 1) {
       const f9::fe left = stack[lvl][threadIdx.x];
       f9::hash2(left, v, C.hk, v);

@@ -1,6 +1,9 @@
 """Weight commitments whose leaf pairs come from the table of int8-range pairs (csrc/merkle.h): the
 matrices are large enough for the table to be used, and mix pairs inside and outside its range, odd row
-counts (a padding leaf beside a real one), padded columns and single-row grids.  Against the oracle."""
+counts (a padding leaf beside a real one), padded columns and single-row grids.  Against the oracle.
+And the time: a matrix that is partly in the range must not take longer than one that is all outside."""
+import time
+
 import numpy as np
 import pytest
 
@@ -56,3 +59,25 @@ def test_with_and_without_the_table(ctx):
     plain = G.Context(0)
     assert ctx.weight_commitment(ctx.upload(m)) == plain.weight_commitment(plain.upload(m))
     plain.close()
+
+
+def test_partly_in_range_takes_no_longer(ctx):
+    """Lanes with a pair in the table and lanes without stay in step: the hashes of a wave are then at most
+    those of a matrix outside the range.  Out of step the mixed one took 1.4 to 2.7 times as long."""
+    rng = np.random.default_rng(4)
+    other = rng.integers(1 << 20, 1 << 30, size=(2048, 2048)).astype(np.uint32)
+    small = rng.integers(0, 128, size=other.shape).astype(np.uint32)
+
+    def best(m):
+        w, ts = ctx.upload(m), []
+        for _ in range(5):
+            w.invalidate()
+            t = time.perf_counter()
+            ctx.weight_commitment(w)
+            ts.append(time.perf_counter() - t)
+        return min(ts)
+
+    outside = best(other)
+    for share in (0.05, 0.5, 0.9):
+        mixed = best(np.where(rng.random(other.shape) < share, other, small))
+        assert mixed < 1.2 * outside, (share, mixed, outside)
