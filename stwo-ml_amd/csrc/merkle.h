@@ -150,8 +150,11 @@ __device__ __forceinline__ void merkle_child(const MerkleStep& T, uint32_t s, ui
 
 // Leaf-pair table: entry (x + 127) * 255 + (y + 127) is H(leaf x, leaf y).
 constexpr uint32_t kPairSide = 255, kPairCount = kPairSide * kPairSide;
-// index of a canonical M31 value on one side of the table, kPairSide or more for none
-__device__ __forceinline__ uint32_t pair_side(uint32_t v) { return v <= 127u ? v + 127u : v - (P - 127u); }
+// index of a matrix value on one side of the table, kPairSide for none
+__device__ __forceinline__ uint32_t pair_side(uint32_t v) {
+  const uint32_t neg = v - (P - 127u);
+  return v <= 127u ? v + 127u : neg < 127u ? neg : kPairSide;
+}
 
 static __global__ void __launch_bounds__(64) k_merkle_pair_table(const MerkleConsts* __restrict__ C,
                                                           f9::fe* __restrict__ table) {

@@ -1,9 +1,11 @@
 """Shared pytest setup: markers, import paths and the built libraries."""
+import ctypes
 import json
 import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -37,3 +39,19 @@ def gpu_ctx():
     ctx = G.Context(0)
     yield ctx
     ctx.close()
+
+
+@pytest.fixture(scope="session")
+def write_words(gpu_ctx):
+    """write_words(matrix, index, words): a matrix's device memory written from outside the library, as a
+    program that owns the memory may (the library's own upload refuses words that are not canonical)."""
+    copy = ctypes.CDLL("libamdhip64.so.7").hipMemcpy  # the runtime the library has loaded
+    copy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+
+    def write(matrix, index, words):
+        w = np.array(words, dtype=np.uint32)
+        assert index + len(w) <= matrix.rows * matrix.cols
+        host_to_device = 1
+        assert copy(matrix.device_ptr + 4 * index, w.ctypes.data, w.nbytes, host_to_device) == 0
+
+    return write

@@ -81,3 +81,15 @@ def test_partly_in_range_takes_no_longer(ctx):
     for share in (0.05, 0.5, 0.9):
         mixed = best(np.where(rng.random(other.shape) < share, other, small))
         assert mixed < 1.2 * outside, (share, mixed, outside)
+
+
+def test_words_past_the_field_are_hashed_as_they_are(ctx, write_words):
+    """P and the words above it are no entries of the table: they keep the leaf of their own word."""
+    w = ctx.upload(np.zeros((64, 64), dtype=np.uint32))
+    zero = ctx.weight_commitment(w)
+    write_words(w, 3 * 64 + 5, [P])
+    w.invalidate()
+    plain = G.Context(0)
+    got = ctx.weight_commitment(w)
+    assert got == plain.weight_commitment(plain.wrap_device(w.device_ptr, 64, 64)) and got != zero
+    plain.close()
