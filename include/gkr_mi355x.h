@@ -142,8 +142,16 @@ int gkr_ctx_reset_timing(gkr_ctx* ctx);
  *     its values: a sumcheck trip's challenges, or an activation layer's
  *     gamma and beta when its first kernels were launched ahead (that wait
  *     expires).
+ *   GKR_DEBUG_REFUSE_LAUNCH (of any call, not only hand-overs): the arg-th next
+ *     kernel launch of the context asks for a workgroup larger than the
+ *     runtime takes; the runtime refuses it and the kernel does not run.
  * Every kernel exits normally and the context stays usable.                 */
-enum { GKR_DEBUG_HANDOVER_CANCEL = 1, GKR_DEBUG_HANDOVER_EXPIRE = 2, GKR_DEBUG_TRIP_EXPIRE = 3 };
+enum {
+  GKR_DEBUG_HANDOVER_CANCEL = 1,
+  GKR_DEBUG_HANDOVER_EXPIRE = 2,
+  GKR_DEBUG_TRIP_EXPIRE = 3,
+  GKR_DEBUG_REFUSE_LAUNCH = 4
+};
 int gkr_ctx_debug(gkr_ctx* ctx, int op, uint64_t arg);
 
 /* ------------------------------------------------------------------ resident matrices

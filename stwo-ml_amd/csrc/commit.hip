@@ -61,10 +61,11 @@ static int merkle_pairs(gkr_ctx* c, const MerkleConsts* K, uint64_t leaf_parents
     f9::fe* d = nullptr;
     HIP_TRY(hipMalloc(&d, kPairCount * sizeof(f9::fe)));
     GKR_LAUNCH(c, k_merkle_pair_table, dim3((kPairCount + 63) / 64), dim3(64), 0, K, d);
-    if (hipGetLastError() != hipSuccess) {
-      drain(c);
+    drain(c);  // kept only once its launch is known to have been taken
+    const int rc = check_launch(c);
+    if (rc != GKR_OK) {
       (void)hipFree(d);
-      return fail(GKR_ERR_DEVICE, "leaf-pair table launch failed");
+      return rc;
     }
     c->merkle_pairs = d;
   }
@@ -202,7 +203,7 @@ static int merkle_roots(gkr_ctx* c, const std::vector<MerkleTreeSpec>& trees, gk
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(roots, dwords, nt * 32, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  return GKR_OK;
+  return check_launch(c);
 }
 
 static int weight_tree(const gkr_matrix* m, MerkleTreeSpec* t) {

@@ -289,6 +289,7 @@ struct gkr_ctx {
   bool debug_handover_cancel = false;  // the host leaves before posting the challenges
   uint32_t debug_handover_spins = 0;   // nonzero: the kernel's bounded wait, posted only after it expired
   uint32_t debug_trip_spins = 0;       // the same for the next trip launched ahead of its challenges
+  uint64_t debug_refuse_launch = 0;    // nonzero: the runtime refuses this launch from now (1: the next)
   // set when a call failed because a kernel's bounded wait for the host gave
   // up (the host fell more than the wait's length behind); the walk then
   // proves the step again
@@ -329,8 +330,12 @@ int ensure_host_mult(gkr_ctx* c, uint64_t n);
 // converted to the kernel's parameter types at this point; the launch itself
 // is issued by the context's launcher thread when it has one.
 #define GKR_LAUNCH(ctx, KERN_, GRID_, BLOCK_, SHMEM_, ...)                                     \
-  (void)launch_kernel((ctx)->launcher.get(), take_armed(ctx), KERN_, dim3(GRID_), dim3(BLOCK_), \
-                      (uint32_t)(SHMEM_), (ctx)->stream, __VA_ARGS__)
+  (void)launch_kernel((ctx)->launcher.get(), take_armed(ctx), KERN_, dim3(GRID_),              \
+                      launch_block(ctx, dim3(BLOCK_)), (uint32_t)(SHMEM_), (ctx)->stream, __VA_ARGS__)
+inline dim3 launch_block(gkr_ctx* c, dim3 block) {
+  if (c->debug_refuse_launch && --c->debug_refuse_launch == 0) return dim3(1u << 16);  // test hook: refused
+  return block;
+}
 // The events a TimedLaunch armed for the next launch (consumed by it).
 inline LaunchEvents take_armed(gkr_ctx* c) {
   const LaunchEvents ev = c->armed;

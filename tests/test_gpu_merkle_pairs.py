@@ -61,6 +61,24 @@ def test_with_and_without_the_table(ctx):
     plain.close()
 
 
+@pytest.mark.parametrize("launch", [1, 2, 3])
+def test_refused_launch(launch):
+    """A launch of the commitment that the runtime refuses (the table's, a level's, the next) fails the call,
+    and nothing of it is kept: the same call then gives the root."""
+    c, m = G.Context(0), O.synthetic(1024, 512, 1, 5)
+    w = c.upload(m)
+    c.debug(G.DEBUG_REFUSE_LAUNCH, launch)
+    with pytest.raises(G.GkrError):
+        c.weight_commitment(w)
+    root = c.weight_commitment(w)
+    small = edges(64, 33, 2)  # below the size that builds the table: the kept one, if any
+    assert c.weight_commitment(c.upload(small)) == O.weight_commitment(small)
+    plain = G.Context(0)
+    assert root == plain.weight_commitment(plain.upload(m))
+    plain.close()
+    c.close()
+
+
 def test_partly_in_range_takes_no_longer(ctx):
     """Lanes with a pair in the table and lanes without stay in step: the hashes of a wave are then at most
     those of a matrix outside the range.  Out of step the mixed one took 1.4 to 2.7 times as long."""
