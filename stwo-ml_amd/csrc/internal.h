@@ -425,8 +425,9 @@ int sync(gkr_ctx* c);
 inline int check_launch(gkr_ctx* c) {
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && c && c->launcher) e = c->launcher->take_error();
-  if (e != hipSuccess) return fail(GKR_ERR_DEVICE, "kernel launch: %s", hipGetErrorString(e));
-  return GKR_OK;
+  if (e == hipSuccess) return GKR_OK;
+  if (c) c->trip_count_valid = false;  // a launch that did not run has not counted its workgroups
+  return fail(GKR_ERR_DEVICE, "kernel launch: %s", hipGetErrorString(e));
 }
 static inline unsigned grid_for(uint64_t n, uint64_t per_block = kBlock) {
   uint64_t g = (n + per_block - 1) / per_block;

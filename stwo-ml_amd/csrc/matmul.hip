@@ -1174,7 +1174,7 @@ extern "C" int gkr_sumcheck_product_noalloc(gkr_ctx* c, const gkr_qm31* fa, cons
                                   final_b);
   c->noalloc = false;
   c->trip_count = saved_count;
-  c->trip_count_valid = saved_valid;
+  c->trip_count_valid = saved_valid && rc == GKR_OK;  // the error may be of a launch before this call
   c->timing = saved_timing;
   const int rs = sync(c);  // nothing of this call still touches the scratch array when the lock is released
   return rc != GKR_OK ? rc : rs;
