@@ -584,7 +584,13 @@ static int prove_norm_core(gkr_ctx* c, bool ln, bool fresh, const gkr_qm31* clai
   PoseidonChannel& C = ch->ch;
   NormReady R;
   TRY(norm_setup(c, X, ln, dim, gamma, ng, d_gamma, z.data(), (int)z.size(), &R));
-  if (R.bad_gamma) return fail(GKR_ERR_INVALID, "gamma holds a value that is not canonical");
+  if (R.bad_gamma) {  // a resident scale: the values are read back to name the first one
+    std::vector<uint32_t> g(ng);
+    HIP_TRY(hipMemcpyAsync(g.data(), d_gamma, ng * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    TRY(sync(c));
+    const uint64_t i = std::find_if(g.begin(), g.end(), [](uint32_t v) { return v >= P; }) - g.begin();
+    return fail(GKR_ERR_INVALID, "gamma value %llu not canonical", (unsigned long long)i);
+  }
   const NormShape& S = R.S;
   const qm31 input_eval = R.input_eval, output_eval = R.output_eval;
   if (fresh) {

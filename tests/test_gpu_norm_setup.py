@@ -1,6 +1,7 @@
 """The norm layers' device pass (csrc/norm.hip: statistics, vectors and evaluations without a host round
 trip) at shapes around its workgroups, and walk steps whose scale is a resident matrix: a fresh claim
-proved from the same pass, a scale longer and shorter than the width, and one that is not canonical."""
+proved from the same pass, a scale longer and shorter than the width, and one that is not canonical, on
+the host (refused before any launch) and resident (found by the device pass)."""
 import numpy as np
 import pytest
 
@@ -57,7 +58,26 @@ def test_scale_not_canonical(gpu_ctx):
     x = gpu_ctx.synthetic(4, 16, 1, 3)
     g = np.ones(16, dtype=np.uint32)
     g[11] = P
-    raw = gpu_ctx.upload(np.ones((1, 16), dtype=np.uint32))
-    with pytest.raises(G.GkrError, match="not canonical"):
+    with pytest.raises(G.GkrError, match="gamma value 11 not canonical"):
         gpu_ctx.prove_norm_layer(G.STEP_RMSNORM, [(0, 0, 0, 0)] * 6, (0, 0, 0, 0), x, 16, G.PoseidonChannel(), gamma=g)
-    G.prove_walk(gpu_ctx, G.PoseidonChannel(), [(G.STEP_RMSNORM, G.CLAIM_FRESH, x, raw, 0, 0, 16)], G.Proof())
+
+
+@pytest.mark.parametrize("claim", [G.CLAIM_FRESH, G.CLAIM_CHAINED])
+@pytest.mark.parametrize("ng,at,bad", [(16, 0, P), (16, 11, P), (40, 39, 0xFFFFFFFF), (200, 199, P), (200, 64, P + 1)])
+def test_resident_scale_not_canonical(gpu_ctx, write_words, claim, ng, at, bad):
+    """A walk's scale is checked where it is: inside the width (16 columns), past it, and past the padded
+    matrix (64 entries); the first bad value is named, and a good scale in its place is then accepted."""
+    x = gpu_ctx.synthetic(4, 16, 1, 3)
+    good = np.full((1, ng), 7, dtype=np.uint32)
+    g = gpu_ctx.upload(good)
+    write_words(g, at, [bad] * (ng - at))
+    step = [(G.STEP_RMSNORM, claim, x, g, 0, 0, 16)]
+    start = dict(init_point=[(1, 2, 3, 4)] * 6, init_value=(1, 0, 0, 0)) if claim == G.CLAIM_CHAINED else {}
+    with pytest.raises(G.GkrError, match="gamma value %d not canonical" % at):
+        G.prove_walk(gpu_ctx, G.PoseidonChannel(), step, G.Proof(), **start)
+    write_words(g, at, good[0, at:])
+    ch, ref = G.PoseidonChannel(), G.PoseidonChannel()
+    up = gpu_ctx.upload(good)
+    got = G.prove_walk(gpu_ctx, ch, step, G.Proof(), **start)
+    assert got == G.prove_walk(gpu_ctx, ref, [step[0][:3] + (up,) + step[0][4:]], G.Proof(), **start)
+    assert ch.digest() == ref.digest()
