@@ -49,9 +49,10 @@ GKR_HD RowStat row_stat(bool layernorm, uint32_t s1, uint32_t s2, uint32_t act, 
 // 4r+3] in host memory; (mean or 0, rsqrt) to rowv[2r .. 2r+1].  Rows past the
 // matrix are zero.  Bound by a row's chain of loads: four in flight per thread,
 // and 1024 threads where a row has work for them; many or short rows take a
-// wave each, which also keeps grids below 2^32 threads.
+// wave each.  A launch takes fewer than 2^32 threads: up to kNormMaxRows padded
+// rows.
 constexpr int kNormRowBlock = 1024;
-constexpr uint64_t kNormWideRows = 1ull << 16;
+constexpr uint64_t kNormWideRows = 1ull << 16, kNormMaxRows = 1ull << 25;
 inline int norm_row_block(uint64_t rows, uint64_t cols) {
   return cols >= kNormRowBlock && rows <= kNormWideRows ? kNormRowBlock : 64;
 }
@@ -201,6 +202,7 @@ int norm_setup(gkr_ctx* c, const gkr_matrix* X, bool ln, uint64_t dim, const uin
   if (S->nv == 0) return fail(GKR_ERR_INVALID, "norm layer over a single entry has no rounds");
   if (dim == 0) return fail(GKR_ERR_INVALID, "norm layer with no active column");
   if (S->nv > kMaxVars) return fail(GKR_ERR_INVALID, "norm layer too large");
+  if (S->prow > kNormMaxRows) return fail(GKR_ERR_INVALID, "norm layer of %llu rows", (unsigned long long)S->rows);
   if (n_z != S->nv) return fail(GKR_ERR_INVALID, "point has %d vars, the norm MLE has %d", n_z, S->nv);
   if (S->n != (1ull << S->nv)) return fail(GKR_ERR_DEVICE, "norm vectors of %llu entries over %d variables",
                                            (unsigned long long)S->n, S->nv);

@@ -81,3 +81,10 @@ def test_resident_scale_not_canonical(gpu_ctx, write_words, claim, ng, at, bad):
     got = G.prove_walk(gpu_ctx, ch, step, G.Proof(), **start)
     assert got == G.prove_walk(gpu_ctx, ref, [step[0][:3] + (up,) + step[0][4:]], G.Proof(), **start)
     assert ch.digest() == ref.digest()
+
+
+def test_more_rows_than_a_launch_takes(gpu_ctx):
+    """2^25 + 1 rows pad to 2^26, whose waves a launch does not take: refused before anything is launched."""
+    x = gpu_ctx.synthetic((1 << 25) + 1, 1, 1, 3)
+    with pytest.raises(G.GkrError, match="norm layer of 33554433 rows"):
+        gpu_ctx.norm_output_claim(G.STEP_RMSNORM, x, 1, [(1, 0, 0, 0)] * 26)
