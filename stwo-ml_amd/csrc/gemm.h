@@ -94,7 +94,7 @@ static __global__ void __launch_bounds__(256) k_digit_mask(const uint32_t* __res
 // outer x K row-major (A: outer = row); kmajor = true: X is K x outer
 // row-major (B: outer = column).  One thread fills one lane slot (16 bytes
 // per plane) of one block; K and outer beyond the matrix are zero.  When mask
-// is given (zero before the launch), bit p is set if plane p is non-zero, and
+// is given (zero before the launch), bit p of 1..3 is set if plane p is non-zero, and
 // *clear, the mask word of the next product on the stream, is zeroed.  VEC
 // (row-major X, K a multiple of 4, X 16-byte aligned): a slot's 16 values are
 // four 16-byte loads (a whole 512 x 5120 x 1024 product 34.0 -> 30.3 us).
@@ -245,7 +245,8 @@ __device__ __forceinline__ void gemm_tile(const int8_t* __restrict__ Ap, uint64_
 // cache delivers; 4 x 2 tiles read 0.75 KB.  The next step's blocks are loaded
 // while this step's are multiplied; every tile shape sums the same integers.
 // Workgroups that share column tiles (the row groups of one column group) are
-// 8 apart in blockIdx, that is on one XCD, whose L2 then reads B once.
+// xcds = 8 apart in blockIdx, that is on one XCD, whose L2 then reads B once
+// (xcds = 1: fewer column groups than XCDs, neighbours in blockIdx).
 // An A with higher planes (*amask) is for gemm_tile: here where a wave has one
 // tile, else in k_gemm_a4, launched behind (one of the two returns at once).
 template <int RT, int CT, int WR>
@@ -253,12 +254,12 @@ static __global__ void __launch_bounds__(256) k_gemm_int8(const int8_t* __restri
                                                    const uint32_t* __restrict__ amask,
                                                    const int8_t* __restrict__ Bp, uint64_t m, uint64_t n,
                                                    uint32_t nsteps, uint32_t rtiles, uint32_t ctiles, uint32_t rgroups,
-                                                   uint32_t cgroups, uint32_t steps_per_split,
+                                                   uint32_t cgroups, uint32_t xcds, uint32_t steps_per_split,
                                                    uint32_t* __restrict__ out) {
   constexpr int WC = 4 / WR;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-  const uint32_t cg = (idx / rgroups) * 8 + xcd, rg = idx % rgroups;
+  const uint32_t xcd = blockIdx.x % xcds, idx = blockIdx.x / xcds;
+  const uint32_t cg = (idx / rgroups) * xcds + xcd, rg = idx % rgroups;
   if (cg >= cgroups) return;
   const uint32_t rt0 = (rg * WR + wave % WR) * RT, ct0 = (cg * WC + wave / WR) * CT;
   if (rt0 >= rtiles || ct0 >= ctiles) return;

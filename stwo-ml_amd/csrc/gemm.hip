@@ -94,16 +94,29 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
     bp = ext;
   }
   const uint64_t waves = rtiles * ctiles, blocks_x = (waves + 3) / 4;
-  // Int8-range operands: the wave's tiles by the rows there are (times of one
-  // product with 5120 x 13824 int8 weights, one tile per wave and 2048
-  // workgroups by K splits before -> now): 4 x 2 from 8 row tiles (m = 512:
-  // 218.5 -> 58.2 us, 1024: 397 -> 104), 2 x 2 from 4 (128 x 5120 x 5120: 42.9
-  // -> 25.0), 2 x 1 from 2 (m = 64: 48.6 -> 32.2), 1 x 1 for one (m = 1: 26.3
-  // -> 19.0).  K is split only where the tiles alone give under 576 waves, and
-  // then into about 768 waves (512 and 1024 up to 1.3 times slower for one
-  // shape or another): a split writes and reads its partial sums.
-  const int RT = rtiles >= 8 ? 4 : rtiles >= 2 ? 2 : 1, CT = rtiles >= 4 ? 2 : 1, WR = rtiles >= 4 ? 2 : 1;
+  // Int8-range operands: the wave's tiles by the work there is, counted in steps
+  // of one 32 x 32 tile of C by 32 of K.  A call of few steps is bound by latency
+  // and launches: one tile per wave, which needs no k_gemm_a4 behind it (us per
+  // call with one tile and with the wider ones: 512 x 576 x 1536 24.3, 34.0; 1024 x
+  // 64 x 64 22.2, 29.5; 256 x 2048 x 2048 29.7, 40.7; 64 x 5120 x 1024 29.1, 33.9).
+  // Above, wider tiles read fewer operands (one tile per wave in 2048 workgroups by
+  // K splits before -> now, weights of 5120 x 13824): 4 x 2 from 8 row tiles (m =
+  // 512: 233.5 -> 66.4), 2 x 2 from 4 (m = 128: 84.9 -> 43.4), 2 x 1 from 2 (m =
+  // 64: 62.9 -> 42.0), 1 x 1 for one (m = 1: 42.0 -> 29.6).  The lines, by one tile
+  // and wider for A of one plane and of four: from 4 row tiles 2^18 steps (256 x
+  // 5120 x 5120, 204,800 steps: 44.0, 49.1 and 101.5, 110.4; 512 x 5120 x 13824,
+  // 1,105,920: 96.7, 69.7 and 313, 322), below 2^16 (64 x 5120 x 5120, 51,200:
+  // 30.9, 37.1 and 49.7, 48.9; 64 x 5120 x 13824, 138,240: 33.0, 42.0 and 85.6,
+  // 68.4).  K is split only where the tiles alone give under 576 waves, and then
+  // into about 768 waves (512 and 1024 up to 1.3 times slower for one shape or
+  // another): a split writes and reads its partial sums.
+  const bool wide = waves * nsteps >= (rtiles >= 4 ? 1ull << 18 : 1ull << 16);
+  const int RT = !wide ? 1 : rtiles >= 8 ? 4 : rtiles >= 2 ? 2 : 1, CT = wide && rtiles >= 4 ? 2 : 1;
+  const int WR = wide && rtiles >= 4 ? 2 : 1;
   const uint64_t rgroups = (rtiles + RT * WR - 1) / (RT * WR), cgroups = (ctiles + CT * (4 / WR) - 1) / (CT * (4 / WR));
+  // column groups to XCDs in turn; few of them would leave XCDs idle, so then
+  // every workgroup goes to the next XCD (4096 x 5120 x 64: 107.7 -> 50.7 us)
+  const uint64_t xcds = cgroups >= 8 ? 8 : 1, blocks8 = (cgroups + xcds - 1) / xcds * xcds * rgroups;
   const uint64_t tile_waves = (rtiles + RT - 1) / RT * ((ctiles + CT - 1) / CT);
   uint64_t splits = PB == 1 ? (tile_waves >= 576 ? 1 : (768 + tile_waves - 1) / tile_waves)
                             : (2048 + blocks_x - 1) / blocks_x;
@@ -111,15 +124,15 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
   splits = std::max<uint64_t>(splits, (nsteps * kGemmK + kGemmMaxKPass - 1) / kGemmMaxKPass);
   const uint64_t sps = (nsteps + splits - 1) / splits;
   splits = (nsteps + sps - 1) / sps;
-  if (blocks_x > 0x7fffffffull || (cgroups + 7) / 8 * 8 * rgroups > 0x7fffffffull || nsteps > 0xffffffffull || splits > 65535)
+  if (blocks_x > 0x7fffffffull || blocks8 > 0x7fffffffull || nsteps > 0xffffffffull || splits > 65535)
     return fail(GKR_ERR_INVALID, "forward GEMM: grid too large");
   uint32_t* part = C;
   if (splits > 1) TRY(ensureT(c, S_GEMMP, splits * m * n, &part));
   if (PB == 1) {
-    const dim3 g8((uint32_t)((cgroups + 7) / 8 * 8 * rgroups), (uint32_t)splits);
+    const dim3 g8((uint32_t)blocks8, (uint32_t)splits);
     auto int8_launch = [&](auto kernel) {
       GKR_LAUNCH(c, kernel, g8, dim3(256), 0, ap, a_plane, amask, bp, m, n, (uint32_t)nsteps, (uint32_t)rtiles,
-                 (uint32_t)ctiles, (uint32_t)rgroups, (uint32_t)cgroups, (uint32_t)sps, part);
+                 (uint32_t)ctiles, (uint32_t)rgroups, (uint32_t)cgroups, (uint32_t)xcds, (uint32_t)sps, part);
     };
     if (RT == 4)
       int8_launch(k_gemm_int8<4, 2, 2>);

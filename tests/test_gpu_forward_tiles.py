@@ -1,6 +1,9 @@
 """The forward product over int8-range weights around its tile shapes (csrc/gemm.h): row counts on both
-sides of each rule (1, 2, 4 and 8 row tiles of 32), ragged columns and inner sizes with and without K
-splits, and activations of one digit plane and of four.  Against exact integers."""
+sides of each rule (1, 2, 4 and 8 row tiles of 32; few and many tile steps), ragged columns and inner
+sizes with and without K splits, and activations of one digit plane and of four.  Against exact integers.
+And the time of products with little work or few columns, by products that do more."""
+import time
+
 import numpy as np
 import pytest
 
@@ -39,14 +42,46 @@ def test_tile_rules(ctx, m, k, n):
     assert np.array_equal(ctx.matmul_forward(ctx.upload(a), dev).download(), exact(a, b))
 
 
+# many tile steps, so that wider tiles than one per wave are taken: 4 x 2, 2 x 2 and 2 x 1, each with
+# its last tiles past the matrix's edges
+@pytest.mark.parametrize("m,k,n", [(513, 3900, 4099), (200, 9400, 4099), (33, 8200, 4099)])
+def test_wide_tiles(ctx, m, k, n):
+    b = O.synthetic(k, n, 1, 7)
+    b[0, 0], b[-1, -1] = 127, P - 127
+    dev = ctx.upload(b)
+    for kind in (1, 0):
+        a = O.synthetic(m, k, kind, 11 + m)
+        assert np.array_equal(ctx.matmul_forward(ctx.upload(a), dev).download(), exact(a, b))
+
+
 def test_one_high_value_takes_the_general_path(ctx):
-    """A single entry of A outside the int8 range, in the last row."""
-    a, b = O.synthetic(300, 200, 1, 5), O.synthetic(200, 300, 1, 6)
-    a[-1, -1] = 1 << 20
-    assert np.array_equal(ctx.matmul_forward(ctx.upload(a), ctx.upload(b)).download(), exact(a, b))
+    """A single entry of A outside the int8 range, in the last row: one tile per wave and wider ones."""
+    for m, k, n in ((300, 200, 300), (257, 4000, 7500)):
+        a, b = O.synthetic(m, k, 1, 5), O.synthetic(k, n, 1, 6)
+        a[-1, -1] = 1 << 20
+        assert np.array_equal(ctx.matmul_forward(ctx.upload(a), ctx.upload(b)).download(), exact(a, b))
 
 
 def test_four_planes_two_column_tiles_per_wave(ctx):
-    """33 x 129 tiles: enough for two column tiles per wave, the last wave's second one past the edge."""
-    a, b = O.synthetic(1030, 40, 0, 8), O.synthetic(40, 4099, 1, 9)
+    """33 x 129 tiles of many steps: enough for two column tiles per wave, the last wave's second one past
+    the edge."""
+    a, b = O.synthetic(1030, 2000, 0, 8), O.synthetic(2000, 4099, 1, 9)
     assert np.array_equal(ctx.matmul_forward(ctx.upload(a), ctx.upload(b)).download(), exact(a, b))
+
+
+def test_small_products_are_not_slowed_by_wide_tiles(ctx):
+    """512 rows of few tile steps take about as long as 32 rows (latency and launches; 1.4 times with tiles
+    of 4 x 2), and 64 columns less than 700 (on one XCD of eight they took longer)."""
+
+    def best(m, k, n):
+        a, b, o, ts = ctx.synthetic(m, k, 1, 3), ctx.synthetic(k, n, 1, 4), ctx.synthetic(m, n, 1, 5), []
+        for _ in range(60):
+            ctx.synchronize()
+            t = time.perf_counter()
+            ctx.matmul_forward_into(a, b, o)
+            ctx.synchronize()
+            ts.append(time.perf_counter() - t)
+        return min(ts)
+
+    assert best(512, 576, 1536) < 1.25 * best(32, 576, 1536)
+    assert best(4096, 5120, 64) < 0.9 * best(4096, 5120, 700)
