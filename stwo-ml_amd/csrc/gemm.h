@@ -238,15 +238,27 @@ __device__ __forceinline__ void gemm_tile(const int8_t* __restrict__ Ap, uint64_
   }
 }
 
+// The row and column group of a workgroup in a grid of gemm_group_blocks(rgroups
+// * cgroups): workgroups of one XCD (blockIdx 8 apart) take a run of the groups,
+// counted down the columns, an eighth of them each, so that those that share
+// column tiles share an L2, which then reads B once, and every XCD has as much
+// to do (column groups to XCDs in turn: 4096 x 5120 x 64 ran on one of the
+// eight, 103.4 us; 50.9 now with one tile per wave).  False: no group.
+__device__ __forceinline__ bool gemm_group(uint32_t rgroups, uint32_t cgroups, uint32_t& rg, uint32_t& cg) {
+  const uint64_t at = (uint64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  rg = (uint32_t)(at % rgroups);
+  cg = (uint32_t)(at / rgroups);
+  return cg < cgroups;
+}
+inline uint64_t gemm_group_blocks(uint64_t groups) { return (groups + 7) / 8 * 8; }
+
 // Int8-range operands (one plane each): a workgroup's 4 waves, WR down and
 // 4 / WR across, each own RT x CT tiles of C, so a K step's RT + CT operand
 // blocks feed RT * CT MFMAs.  One 32 x 32 tile per wave reads 2 KB per MFMA
 // (32 cycles of a SIMD), 256 bytes a cycle and CU against the 64 the vector
 // cache delivers; 4 x 2 tiles read 0.75 KB.  The next step's blocks are loaded
 // while this step's are multiplied; every tile shape sums the same integers.
-// Workgroups that share column tiles (the row groups of one column group) are
-// xcds = 8 apart in blockIdx, that is on one XCD, whose L2 then reads B once
-// (xcds = 1: fewer column groups than XCDs, neighbours in blockIdx).
+// Workgroups go to XCDs by gemm_group.
 // An A with higher planes (*amask) is for gemm_tile: here where a wave has one
 // tile, else in k_gemm_a4, launched behind (one of the two returns at once).
 template <int RT, int CT, int WR>
@@ -254,13 +266,12 @@ static __global__ void __launch_bounds__(256) k_gemm_int8(const int8_t* __restri
                                                    const uint32_t* __restrict__ amask,
                                                    const int8_t* __restrict__ Bp, uint64_t m, uint64_t n,
                                                    uint32_t nsteps, uint32_t rtiles, uint32_t ctiles, uint32_t rgroups,
-                                                   uint32_t cgroups, uint32_t xcds, uint32_t steps_per_split,
+                                                   uint32_t cgroups, uint32_t steps_per_split,
                                                    uint32_t* __restrict__ out) {
   constexpr int WC = 4 / WR;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t xcd = blockIdx.x % xcds, idx = blockIdx.x / xcds;
-  const uint32_t cg = (idx / rgroups) * xcds + xcd, rg = idx % rgroups;
-  if (cg >= cgroups) return;
+  uint32_t rg, cg;
+  if (!gemm_group(rgroups, cgroups, rg, cg)) return;
   const uint32_t rt0 = (rg * WR + wave % WR) * RT, ct0 = (cg * WC + wave / WR) * CT;
   if (rt0 >= rtiles || ct0 >= ctiles) return;
   const uint32_t split = blockIdx.y, s0 = split * steps_per_split;
@@ -323,20 +334,26 @@ static __global__ void __launch_bounds__(256) k_gemm_int8(const int8_t* __restri
     }
 }
 
-// One wave per 32 rows x CT * 32 columns of C and K split: A of four planes by
-// a one-plane B.  CT = 2 loads 0.75 KB per MFMA instead of 1.25 (512 x 5120 x
-// 13824: 333 -> 309 us) and is for products with enough waves left.
+// A of four planes by a one-plane B: one wave per 32 rows x CT * 32 columns of
+// C and K split.  A workgroup's four waves take the same rows, whose four KB a
+// K step they then share in the vector cache, and columns next to each other
+// (four row tiles of one column instead, both before the barrier in
+// gemm_tile: 200 x 13824 x 5120 216 us against 190, 300 x 5120 x 13824 254
+// against 227, 512 x 5120 x 13824 320 against 297).
 template <int CT>
 static __global__ void __launch_bounds__(256) k_gemm_a4(const int8_t* __restrict__ Ap, uint64_t a_plane_bytes,
                                                  const uint32_t* __restrict__ amask, const int8_t* __restrict__ Bp,
-                                                 uint64_t m, uint64_t n, uint64_t nsteps, uint64_t rtiles,
-                                                 uint64_t ctiles, uint64_t steps_per_split, uint32_t* __restrict__ out) {
+                                                 uint64_t m, uint64_t n, uint64_t nsteps, uint32_t rtiles,
+                                                 uint32_t ctiles, uint32_t cgroups, uint64_t steps_per_split,
+                                                 uint32_t* __restrict__ out) {
   if (!(*amask & 0xeu)) return;  // uniform
-  const uint64_t wave = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wave >= rtiles * ((ctiles + CT - 1) / CT)) return;
+  uint32_t rt, cg;
+  if (!gemm_group(rtiles, cgroups, rt, cg)) return;
+  const uint32_t ct = (cg * 4 + (threadIdx.x >> 6)) * CT;
+  if (ct >= ctiles) return;
   const uint64_t s0 = blockIdx.y * steps_per_split;
   const uint64_t s1 = s0 + steps_per_split < nsteps ? s0 + steps_per_split : nsteps;
-  gemm_tile<4, 1, CT, 4>(Ap, a_plane_bytes, Bp, 0, m, n, nsteps, wave % rtiles, wave / rtiles * CT, ctiles, s0, s1,
+  gemm_tile<4, 1, CT, 4>(Ap, a_plane_bytes, Bp, 0, m, n, nsteps, rt, ct, ctiles, s0, s1,
                          out + (uint64_t)blockIdx.y * m * n);
 }
 

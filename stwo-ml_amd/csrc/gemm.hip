@@ -97,29 +97,37 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
   // Int8-range operands: the wave's tiles by the work there is, counted in steps
   // of one 32 x 32 tile of C by 32 of K.  A call of few steps is bound by latency
   // and launches: one tile per wave, which needs no k_gemm_a4 behind it (us per
-  // call with one tile and with the wider ones: 512 x 576 x 1536 24.3, 34.0; 1024 x
-  // 64 x 64 22.2, 29.5; 256 x 2048 x 2048 29.7, 40.7; 64 x 5120 x 1024 29.1, 33.9).
+  // call with one tile and with the wider ones: 512 x 576 x 1536 23.7, 29.0; 512 x
+  // 64 x 64 21.3, 24.4; 256 x 2560 x 5120 32.6, 42.3; 64 x 5120 x 1024 24.2, 28.8).
   // Above, wider tiles read fewer operands (one tile per wave in 2048 workgroups by
   // K splits before -> now, weights of 5120 x 13824): 4 x 2 from 8 row tiles (m =
-  // 512: 233.5 -> 66.4), 2 x 2 from 4 (m = 128: 84.9 -> 43.4), 2 x 1 from 2 (m =
-  // 64: 62.9 -> 42.0), 1 x 1 for one (m = 1: 42.0 -> 29.6).  The lines, by one tile
+  // 512: 232.5 -> 67.4), 2 x 2 from 4 (m = 128: 83.9 -> 43.2), 2 x 1 from 2 (m =
+  // 64: 63.5 -> 42.1), 1 x 1 for one (m = 1: 41.2 -> 29.7).  The lines, by one tile
   // and wider for A of one plane and of four: from 4 row tiles 2^18 steps (256 x
-  // 5120 x 5120, 204,800 steps: 44.0, 49.1 and 101.5, 110.4; 512 x 5120 x 13824,
-  // 1,105,920: 96.7, 69.7 and 313, 322), below 2^16 (64 x 5120 x 5120, 51,200:
-  // 30.9, 37.1 and 49.7, 48.9; 64 x 5120 x 13824, 138,240: 33.0, 42.0 and 85.6,
-  // 68.4).  K is split only where the tiles alone give under 576 waves, and then
-  // into about 768 waves (512 and 1024 up to 1.3 times slower for one shape or
-  // another): a split writes and reads its partial sums.
+  // 5120 x 5120, 204,800 steps: 40.4, 44.8 and 103, 86; 512 x 5120 x 13824,
+  // 1,105,920: 96.8, 66.5 and 302, 258), below 2^16 (64 x 5120 x 5120, 51,200: 27.8,
+  // 32.1 and 45.4, 46.5; 64 x 5120 x 13824, 138,240: 32.6, 41.6 and 65.9, 60.4).
+  // K is split only where the tiles alone give under 576 waves, and then into
+  // about 768 waves (512 and 1024 up to 1.3 times slower for one shape or another):
+  // a split writes and reads its partial sums.  With one tile per wave
+  // of more than 80 steps, up to 5 splits (or of 40 steps) are made for 1536 waves:
+  // a wave's chain of steps is what an A of four planes waits for (in 2048
+  // workgroups, by the rule for 768 waves, now: 1 x 5120 x 13824 49.4, 59.3, 43.2;
+  // 128 x 5120 x 5120 75.8, 70.2, 56.8; 1 x 3000 x 11000 34.2, 39.6, 31.0), and an A
+  // of one plane loses little (1 x 13824 x 5120 30.8 -> 31.5).  For the same reason
+  // chains over 256 steps are halved where the tiles are under 2048 (96 x 13824 x
+  // 13824: 206, 236, 206; A of one plane 129, 108, 76).
   const bool wide = waves * nsteps >= (rtiles >= 4 ? 1ull << 18 : 1ull << 16);
   const int RT = !wide ? 1 : rtiles >= 8 ? 4 : rtiles >= 2 ? 2 : 1, CT = wide && rtiles >= 4 ? 2 : 1;
   const int WR = wide && rtiles >= 4 ? 2 : 1;
   const uint64_t rgroups = (rtiles + RT * WR - 1) / (RT * WR), cgroups = (ctiles + CT * (4 / WR) - 1) / (CT * (4 / WR));
-  // column groups to XCDs in turn; few of them would leave XCDs idle, so then
-  // every workgroup goes to the next XCD (4096 x 5120 x 64: 107.7 -> 50.7 us)
-  const uint64_t xcds = cgroups >= 8 ? 8 : 1, blocks8 = (cgroups + xcds - 1) / xcds * xcds * rgroups;
+  const uint64_t blocks8 = gemm_group_blocks(rgroups * cgroups);
   const uint64_t tile_waves = (rtiles + RT - 1) / RT * ((ctiles + CT - 1) / CT);
   uint64_t splits = PB == 1 ? (tile_waves >= 576 ? 1 : (768 + tile_waves - 1) / tile_waves)
                             : (2048 + blocks_x - 1) / blocks_x;
+  if (PB == 1 && nsteps > 256 * splits && waves * splits < 2048) splits *= 2;
+  if (PB == 1 && RT * CT == 1 && nsteps > 80 && tile_waves < 1024)
+    splits = std::max(splits, std::min<uint64_t>(std::max<uint64_t>(5, nsteps / 40), (1536 + tile_waves - 1) / tile_waves));
   splits = std::min<uint64_t>(splits, std::max<uint64_t>(1, nsteps / 16));
   splits = std::max<uint64_t>(splits, (nsteps * kGemmK + kGemmMaxKPass - 1) / kGemmMaxKPass);
   const uint64_t sps = (nsteps + splits - 1) / splits;
@@ -132,7 +140,7 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
     const dim3 g8((uint32_t)blocks8, (uint32_t)splits);
     auto int8_launch = [&](auto kernel) {
       GKR_LAUNCH(c, kernel, g8, dim3(256), 0, ap, a_plane, amask, bp, m, n, (uint32_t)nsteps, (uint32_t)rtiles,
-                 (uint32_t)ctiles, (uint32_t)rgroups, (uint32_t)cgroups, (uint32_t)xcds, (uint32_t)sps, part);
+                 (uint32_t)ctiles, (uint32_t)rgroups, (uint32_t)cgroups, (uint32_t)sps, part);
     };
     if (RT == 4)
       int8_launch(k_gemm_int8<4, 2, 2>);
@@ -143,11 +151,15 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
     else
       int8_launch(k_gemm_int8<1, 1, 1>);
     auto a4_launch = [&](auto kernel, uint64_t ct) {
-      GKR_LAUNCH(c, kernel, dim3((uint32_t)((rtiles * ((ctiles + ct - 1) / ct) + 3) / 4), (uint32_t)splits), dim3(256), 0,
-                 ap, a_plane, amask, bp, m, n, nsteps, rtiles, ctiles, sps, part);
+      const uint64_t groups = (ctiles + 4 * ct - 1) / (4 * ct);
+      GKR_LAUNCH(c, kernel, dim3((uint32_t)gemm_group_blocks(rtiles * groups), (uint32_t)splits), dim3(256), 0, ap, a_plane,
+                 amask, bp, m, n, nsteps, (uint32_t)rtiles, (uint32_t)ctiles, (uint32_t)groups, sps, part);
     };
-    // two column tiles per wave from 4096 tiles (128 x 1024 x 1024, 128 tiles: 17.9 us with one, 22.2 with two)
-    if (RT * CT > 1 && waves * splits >= 4096)
+    // two column tiles per wave in chains of 80 steps and with columns for every
+    // wave (one, two, us: 64 x 5120 x 13824 67.5, 60.4; 200 x 13824 x 5120 168, 142;
+    // 512 x 8192 x 8192 305, 242; 384 x 3000 x 11000, 47 steps, 133, 147; 16384 x 5120 x
+    // 128, 4 column tiles, 287, 360)
+    if (RT * CT > 1 && ctiles >= 32 && sps >= 80)
       a4_launch(k_gemm_a4<2>, 2);
     else if (RT * CT > 1)
       a4_launch(k_gemm_a4<1>, 1);
