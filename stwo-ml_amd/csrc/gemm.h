@@ -243,19 +243,26 @@ __device__ __forceinline__ void gemm_tile(const int8_t* __restrict__ Ap, uint64_
   }
 }
 
-// The row and column group of a workgroup in a grid of gemm_group_blocks(rgroups
-// * cgroups): workgroups of one XCD (blockIdx 8 apart) take a run of the groups,
+// The row and column group of a workgroup in a grid of gemm_group_grid:
+// workgroups of one XCD (blockIdx 8 apart) take a run of the groups,
 // counted down the columns, an eighth of them each, so that those that share
 // column tiles share an L2, which then reads B once, and every XCD has as much
 // to do (column groups to XCDs in turn: 4096 x 5120 x 64 ran on one of the
-// eight, 103.4 us; 50.9 now with one tile per wave).  False: no group.
+// eight, 103.4 us; 50.9 now with one tile per wave).  blockIdx.z counts runs of
+// rgroups row groups, for grids that a launch would not take in one dimension.
+// False: no group.
 __device__ __forceinline__ bool gemm_group(uint32_t rgroups, uint32_t cgroups, uint32_t& rg, uint32_t& cg) {
   const uint64_t at = (uint64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  rg = (uint32_t)(at % rgroups);
+  rg = (uint32_t)(at % rgroups) + blockIdx.z * rgroups;
   cg = (uint32_t)(at / rgroups);
   return cg < cgroups;
 }
-inline uint64_t gemm_group_blocks(uint64_t groups) { return (groups + 7) / 8 * 8; }
+constexpr uint64_t kGemmMaxGroups = 1ull << 23;  // of 256 threads: half of the 2^32 that a dimension takes
+inline dim3 gemm_group_grid(uint64_t rgroups, uint64_t cgroups, uint64_t splits, uint32_t* rgroups_arg) {
+  const uint64_t z = rgroups * cgroups / kGemmMaxGroups + 1, rows = (rgroups + z - 1) / z;
+  *rgroups_arg = (uint32_t)rows;
+  return dim3((uint32_t)((rows * cgroups + 7) / 8 * 8), (uint32_t)splits, (uint32_t)z);
+}
 
 // Int8-range operands (one plane each): a workgroup's 4 waves, WR down and
 // 4 / WR across, each own RT x CT tiles of C, so a K step's RT + CT operand
@@ -349,13 +356,13 @@ template <int CT>
 static __global__ void __launch_bounds__(256) k_gemm_a4(const int8_t* __restrict__ Ap, uint64_t a_plane_bytes,
                                                  const uint32_t* __restrict__ amask, const int8_t* __restrict__ Bp,
                                                  uint64_t m, uint64_t n, uint64_t nsteps, uint32_t rtiles,
-                                                 uint32_t ctiles, uint32_t cgroups, uint64_t steps_per_split,
-                                                 uint32_t* __restrict__ out) {
+                                                 uint32_t ctiles, uint32_t rgroups, uint32_t cgroups,
+                                                 uint64_t steps_per_split, uint32_t* __restrict__ out) {
   if (!(*amask & 0xeu)) return;  // uniform
   uint32_t rt, cg;
-  if (!gemm_group(rtiles, cgroups, rt, cg)) return;
+  if (!gemm_group(rgroups, cgroups, rt, cg)) return;
   const uint32_t ct = (cg * 4 + (threadIdx.x >> 6)) * CT;
-  if (ct >= ctiles) return;
+  if (rt >= rtiles || ct >= ctiles) return;
   const uint64_t s0 = blockIdx.y * steps_per_split;
   const uint64_t s1 = s0 + steps_per_split < nsteps ? s0 + steps_per_split : nsteps;
   gemm_tile<4, 1, CT, 4>(Ap, a_plane_bytes, Bp, 0, m, n, nsteps, rt, ct, ctiles, s0, s1,

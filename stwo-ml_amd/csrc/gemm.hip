@@ -121,7 +121,6 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
   const int RT = !wide ? 1 : rtiles >= 8 ? 4 : rtiles >= 2 ? 2 : 1, CT = wide && rtiles >= 4 ? 2 : 1;
   const int WR = wide && rtiles >= 4 ? 2 : 1;
   const uint64_t rgroups = (rtiles + RT * WR - 1) / (RT * WR), cgroups = (ctiles + CT * (4 / WR) - 1) / (CT * (4 / WR));
-  const uint64_t blocks8 = gemm_group_blocks(rgroups * cgroups);
   const uint64_t tile_waves = (rtiles + RT - 1) / RT * ((ctiles + CT - 1) / CT);
   uint64_t splits = PB == 1 ? (tile_waves >= 576 ? 1 : (768 + tile_waves - 1) / tile_waves)
                             : (2048 + blocks_x - 1) / blocks_x;
@@ -132,15 +131,16 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
   splits = std::max<uint64_t>(splits, (nsteps * kGemmK + kGemmMaxKPass - 1) / kGemmMaxKPass);
   const uint64_t sps = (nsteps + splits - 1) / splits;
   splits = (nsteps + sps - 1) / sps;
-  if (blocks_x > 0x7fffffffull || blocks8 > 0x7fffffffull || nsteps > 0xffffffffull || splits > 65535)
+  if (blocks_x > 0x7fffffffull || nsteps > 0xffffffffull || splits > 65535)
     return fail(GKR_ERR_INVALID, "forward GEMM: grid too large");
   uint32_t* part = C;
   if (splits > 1) TRY(ensureT(c, S_GEMMP, splits * m * n, &part));
   if (PB == 1) {
-    const dim3 g8((uint32_t)blocks8, (uint32_t)splits);
     auto int8_launch = [&](auto kernel) {
-      GKR_LAUNCH(c, kernel, g8, dim3(256), 0, ap, a_plane, amask, bp, m, n, (uint32_t)nsteps, (uint32_t)rtiles,
-                 (uint32_t)ctiles, (uint32_t)rgroups, (uint32_t)cgroups, (uint32_t)sps, part);
+      uint32_t rg;
+      const dim3 grid = gemm_group_grid(rgroups, cgroups, splits, &rg);
+      GKR_LAUNCH(c, kernel, grid, dim3(256), 0, ap, a_plane, amask, bp, m, n, (uint32_t)nsteps, (uint32_t)rtiles,
+                 (uint32_t)ctiles, rg, (uint32_t)cgroups, (uint32_t)sps, part);
     };
     if (RT == 4)
       int8_launch(k_gemm_int8<4, 2, 2>);
@@ -151,9 +151,11 @@ static int matmul_forward(gkr_ctx* c, const gkr_matrix* a, gkr_matrix* b, uint32
     else
       int8_launch(k_gemm_int8<1, 1, 1>);
     auto a4_launch = [&](auto kernel, uint64_t ct) {
+      uint32_t rg;
       const uint64_t groups = (ctiles + 4 * ct - 1) / (4 * ct);
-      GKR_LAUNCH(c, kernel, dim3((uint32_t)gemm_group_blocks(rtiles * groups), (uint32_t)splits), dim3(256), 0, ap, a_plane,
-                 amask, bp, m, n, nsteps, (uint32_t)rtiles, (uint32_t)ctiles, (uint32_t)groups, sps, part);
+      const dim3 grid = gemm_group_grid(rtiles, groups, splits, &rg);
+      GKR_LAUNCH(c, kernel, grid, dim3(256), 0, ap, a_plane, amask, bp, m, n, nsteps, (uint32_t)rtiles, (uint32_t)ctiles,
+                 rg, (uint32_t)groups, sps, part);
     };
     // two column tiles per wave in chains of 80 steps and with columns for every
     // wave (one, two, us: 64 x 5120 x 13824 67.5, 60.4; 200 x 13824 x 5120 168, 142;

@@ -100,3 +100,16 @@ def test_loads_of_general_weights_are_in_flight_together(ctx):
     """One row by weights of four digit planes reads the weights whatever the row's range, and one plane of it
     has a quarter of the multiplications: 0.86 of a general row's time (0.98 with two loads in flight)."""
     assert best(ctx, 1, 5120, 13824, 1, 0) < 0.93 * best(ctx, 1, 5120, 13824, 0, 0)
+
+
+def test_rows_for_a_grid_of_two_layers():
+    """2^23 + 1 row tiles of one column: the four-plane kernel's workgroups fill two layers of the grid."""
+    m = (1 << 28) + 3
+    c = G.Context(0)
+    a, b = c.synthetic(m, 1, 0, 3), c.upload(np.array([[P - 5]], dtype=np.uint32))
+    got = c.matmul_forward(a, b).download().reshape(-1)
+    x = a.download().reshape(-1)
+    for i in range(0, m, 1 << 25):
+        v = x[i:i + (1 << 25)].astype(np.int64) * -5 % P
+        assert np.array_equal(got[i:i + (1 << 25)], v.astype(np.uint32)), i
+    c.close()
