@@ -608,8 +608,9 @@ int prove_activation(gkr_ctx* c, const gkr_qm31* claim_point, uint32_t n_point, 
   // (4 MB for 2^20 entries take 77 us at the link's rate), each queued where
   // the host draws challenges meanwhile: behind the multiplicity sumcheck's
   // first trip, while it finishes the eq-sumcheck, and behind that sumcheck's
-  // hand-over.  Softmax over 2560 x 64 with the 2^20 table: 622 us with the
-  // whole copy before the first trip, 576 with halves.
+  // hand-over.  Softmax over 2560 x 64 with the 2^20 table, three rounds of both
+  // in turn: 629 to 637 us with the whole copy before the first trip, 573 to
+  // 581 with halves.
   const uint64_t mult_half = tsize / 2;
   auto mult_to_host = [&](int half) -> int {
     GKR_LAUNCH(c, k_u32_to_host, dim3(grid_for(mult_half)), dim3(kBlock), 0, d_mult + half * mult_half, mult_half,

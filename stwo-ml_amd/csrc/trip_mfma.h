@@ -36,10 +36,10 @@
 // card's plain read rate), the second, which reads them again and writes an
 // eighth, 1960 us (4.9 TB/s; its arithmetic alone allows about 4 times that);
 // one round per trip took 8 trips of 848 us.  Whole product sumcheck: 2^28
-// 7174 -> 4070 us, 2^24 735 -> 508, 2^20 266 -> 244, 2^17 202 -> 192.  Tried:
-// cached loads (4.33 ms), four values folded together (4.16), three waves per
-// SIMD (spills, 4.50), 256 or 1024 workgroups, contiguous or XCD-local ranges
-// per workgroup (no faster).  Eq-sumchecks take the two factors of their
+// 6999 -> 3985 us, 2^24 735 -> 508, 2^20 266 -> 244, 2^17 202 -> 192.  Tried,
+// against 4.07 ms at that time: cached loads (4.33 ms), four values folded
+// together (4.16), three waves per SIMD (spills, 4.50), 256 or 1024 workgroups,
+// contiguous or XCD-local ranges per workgroup (no faster).  Eq-sumchecks take the two factors of their
 // weight one on each side: the Mul layer of 64 x 13824 (2^20 entries, four
 // trips instead of five) 330 -> 309 us, two RMSNorm layers of 64 x 5120 (2^19;
 // Part 0 and Part 1) 2204 -> 2164 us.
