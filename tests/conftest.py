@@ -19,7 +19,7 @@ ORACLE_SO = os.path.join(ROOT, "oracle", "_build", "liboracle.so")
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (HIP device)")
-    # Build what is missing (in the build container; the GPU box receives
+    # Build what is missing (where there is a compiler; other machines receive
     # the libraries prebuilt).
     if not os.path.exists(ORACLE_SO):
         subprocess.run(["make", "-C", os.path.join(ROOT, "oracle")], check=True)
